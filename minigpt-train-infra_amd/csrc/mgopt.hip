@@ -58,11 +58,17 @@ constexpr int kUnroll = 1;           // 4-element accesses in flight per thread 
 constexpr bool kNtLoad = true;       // nontemporal loads of grad/param/exp_avg/exp_avg_sq
 constexpr bool kNtStore = true;      // nontemporal stores of param/exp_avg/exp_avg_sq
 // Pass-1 accesses in flight per thread, and elements per access of 16-bit
-// gradients (fp32 gradients take 4, one 16-B access).  Unrolls of 4 and 8
-// and 16-B accesses of eight 16-bit values measured no faster on GPT-2-small
-// (0.053 ms), and 16-B accesses 7-8 % slower on the Qwen3-8B set's bf16
-// gradients (2.47-2.51 ms against 2.31).
-constexpr int kNormUnroll = 2;
+// gradients (fp32 gradients take 4, one 16-B access).  What bounds pass 1 on a
+// set of one round of work-groups is the latency of each thread's own loads,
+// so four are in flight: traced against two, at the chunks of norm_chunk_for,
+// 5.6 against 6.6 us on 4.2M fp32 gradients, 17.7 against 19.8 us on 38.9M
+// bf16, 8.4 against 9.0 us on 16.8M bf16, 0.721 against 0.766 ms on 20,000
+// ragged tensors (2.5e9 fp16), 380 against 386 us on 1.3e9 bf16.  16-B
+// accesses of eight 16-bit values, two or four in flight, landed within 2 % of
+// that up to 1.3e9 elements (17.8-19.3, 8.6-9.0 us, 0.72-0.74 ms, 391-393 us)
+// and were 7-8 % slower on the Qwen3-8B set's bf16 gradients (2.47-2.51 ms
+// against 2.31).
+constexpr int kNormUnroll = 4;
 constexpr int kNormVec16 = 4;
 // Pass 2 reads the gradients pass 1 has just read.  When a plan's gradients
 // fit in the MI355X's 256 MB Infinity Cache (the memory-side cache in front
@@ -74,16 +80,25 @@ constexpr int kNormVec16 = 4;
 // 2.6 GB and 16 GB gradient sets, with no gain in pass 2 beyond run-to-run
 // spread.  Nontemporal pass-2 gradient loads still hit the cache.
 constexpr int64_t kCachedGradBytes = int64_t(256) << 20;
-// pass 1 has its own chunk table of kNormChunk elements per chunk and
-// work-group, whatever the pass-2 chunk size: the finalize kernel then reads
-// one partial per 128K elements.  Pass 1 + finalize measured in one process
-// on the Qwen3-8B set: 16K-element chunks 2.94 ms, 32K 2.50, 64K 2.35,
-// 128K 2.29, 256K 2.31, 512K 2.31; above 128K the smaller sets lose (GPT-2
-// small 0.049 ms at 128K, 0.100 at 512K).  Smaller chunks on small sets
-// (the largest power of two down to 16K giving 2048 work-groups: 32K on
-// GPT-2-small, 16K on the 0.8M set) measured the same (0.047 ms, 0.015 ms).
+// pass 1 has its own chunk table, whatever the pass-2 chunk size: at most
+// kNormChunk elements per chunk and work-group, so that the finalize kernel
+// reads one partial per 128K elements on a large set.  Pass 1 + finalize
+// measured in one process on the Qwen3-8B set: 16K-element chunks 2.94 ms, 32K
+// 2.50, 64K 2.35, 128K 2.29, 256K 2.31, 512K 2.31.
+// A smaller set's chunks shrink, down to kNormChunkMin, until it has
+// kNormGroups of them (norm_chunk_for): 128K-element chunks leave 4.2M
+// gradients on 32 of the 256 CUs.  Pass 1 + finalize traced at 128K / 64K /
+// 32K / 16K / 8K elements per chunk: 4.2M fp32 16.2+3.8 / 10.1+3.9 / 6.5+2.1 /
+// 5.6+2.1 / 5.6+2.2 us; 16.8M bf16 in one buffer 13.0+3.9 / 8.3+1.9 / 8.7+2.0 /
+// 8.4+2.2 / 10.1+3.9; 38.9M bf16 (GPT, 4 x 512) 25.5+4.8 / 20.3+5.1 / 19.0+5.0
+// / 17.7+5.0 / 20.7+4.8; 124.5M (GPT-2-small) fp32 81+5.0 / 82+5.0 / 77+5.2 /
+// 78+6.3 / 73+9.5, fp16 54+5 / 53+6 / 53+6 / 56+7 / 71+10; 2.5e9 fp16 in 20,000
+// ragged tensors 721+14 / 705+20 / 710+32 / 811+56 / 1081+104.  From 2,048
+// chunks on, the finalize's longer list costs what the shorter chunks gain.
 // A grid-stride form with 1024-4096 work-groups per class was slower still.
 constexpr int64_t kNormChunk = 131072;
+constexpr int64_t kNormChunkMin = 16384;
+constexpr int64_t kNormGroups = 2048;
 // Small plans run a step as three kernels instead of five: pass 1 with the
 // finalize in its last work-group, pass 2 with the prologue folded in, and
 // the scaler update.  A plan qualifies with at most kFoldElems elements, no
@@ -603,15 +618,16 @@ __global__ void __launch_bounds__(kBlock) norm_kernel(const NormArgs a) {
 }
 
 // Pass 1 over one flat gradient buffer: work-group r sums elements
-// [r * kNormChunk, (r + 1) * kNormChunk) into partial r, the chunks and
-// partials a one-tensor plan has.
+// [r * chunk, (r + 1) * chunk) into partial r, the chunks and partials a
+// one-tensor plan has.  16.8M bf16 elements: 8.4 us where fixed 128K-element
+// chunks (129 work-groups, two loads in flight) took 16.4.
 template <typename GT, bool NT>
 __global__ void __launch_bounds__(kBlock)
-    norm_flat_kernel(const GT* __restrict__ g, int64_t n, const float* scale, Partial* partials) {
+    norm_flat_kernel(const GT* __restrict__ g, int64_t n, int64_t chunk, const float* scale, Partial* partials) {
     double acc = 0.0;
     uint32_t bad = 0;
-    const int64_t start = static_cast<int64_t>(blockIdx.x) * kNormChunk;
-    norm_chunk<GT, NT>(g + start, min(kNormChunk, n - start), inv_scale_of(scale), scale != nullptr, acc, bad);
+    const int64_t start = static_cast<int64_t>(blockIdx.x) * chunk;
+    norm_chunk<GT, NT>(g + start, min(chunk, n - start), inv_scale_of(scale), scale != nullptr, acc, bad);
     block_reduce<kBlock>(acc, bad);
     if (threadIdx.x == 0) {
         Partial p;
@@ -1187,7 +1203,7 @@ struct mgopt_plan {
     int64_t n_chunks = 0;
     DevTensor* d_tensors = nullptr;
     Chunk* d_chunks = nullptr;       // pass 2 (and helpers): chunk_elems elements per chunk
-    Chunk* d_norm_chunks = nullptr;  // pass 1: kNormChunk elements per chunk
+    Chunk* d_norm_chunks = nullptr;  // pass 1: norm_chunk elements per chunk
     void** d_grads = nullptr;
     Partial* d_partials = nullptr;
     int* d_flags = nullptr;          // set by the prologue when it computed bias corrections on the device
@@ -1247,13 +1263,24 @@ int launch_norm(const mgopt_plan* P, const mgopt_plan::Class& c, const float* sc
     return 0;
 }
 
+// Elements per pass-1 chunk of a set (kNormChunk above): the largest power of
+// two that gives it kNormGroups chunks, within [kNormChunkMin, kNormChunk].
+// chunks(c) is the set's number of chunks of c elements.
+template <typename F>
+int64_t norm_chunk_for(F chunks) {
+    int64_t c = kNormChunk;
+    while (c > kNormChunkMin && chunks(c) < kNormGroups) c /= 2;
+    return c;
+}
+
 template <typename GT>
-void launch_norm_flat(const void* grads, int64_t n, const float* scale, Partial* part, dim3 grid, hipStream_t s) {
+void launch_norm_flat(const void* grads, int64_t n, int64_t chunk, const float* scale, Partial* part, dim3 grid,
+                      hipStream_t s) {
     const GT* g = static_cast<const GT*>(grads);
     if (n * static_cast<int64_t>(sizeof(GT)) <= kCachedGradBytes)
-        hipLaunchKernelGGL((norm_flat_kernel<GT, false>), grid, dim3(kBlock), 0, s, g, n, scale, part);
+        hipLaunchKernelGGL((norm_flat_kernel<GT, false>), grid, dim3(kBlock), 0, s, g, n, chunk, scale, part);
     else
-        hipLaunchKernelGGL((norm_flat_kernel<GT, true>), grid, dim3(kBlock), 0, s, g, n, scale, part);
+        hipLaunchKernelGGL((norm_flat_kernel<GT, true>), grid, dim3(kBlock), 0, s, g, n, chunk, scale, part);
 }
 
 // The extra arguments of a folded pass 2.
@@ -1301,8 +1328,8 @@ int dtype_size(int32_t dt) {
 // allocation-free norm: partials in a static device array
 // ---------------------------------------------------------------------------
 
-// Partials of mgopt_grad_norm_noalloc, one per 131,072-element chunk: 1 MiB,
-// so one call covers at most 65,536 x 131,072 = 8,589,934,592 elements.  Each
+// Partials of mgopt_grad_norm_noalloc, one per chunk of at most 131,072
+// elements: 1 MiB, so one call covers at most 65,536 x 131,072 = 8,589,934,592 elements.  Each
 // GPU the library runs on holds its own copy until the process ends, and every
 // call on that GPU shares it (calls that overlap on one GPU race).  Every slot
 // a call reads is written by the same call, so nothing needs clearing.
@@ -1404,7 +1431,13 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
     const bool fold_forced = fold_env && std::strcmp(fold_env, "1") == 0;
     const bool fold_fits = total_elems <= kFoldElems && (largest + chunk_elems - 1) / chunk_elems <= kFoldTensorChunks;
     P->fold = total_elems > 0 && !has_empty && !fold_off && (fold_fits || (fold_forced && total_elems <= kFoldForcedElems));
-    P->norm_chunk = P->fold ? kNormChunkFold : kNormChunk;
+    P->norm_chunk = kNormChunkFold;
+    if (!P->fold)
+        P->norm_chunk = norm_chunk_for([&](int64_t c) {
+            int64_t k = 0;
+            for (int32_t i = 0; i < n_tensors; ++i) k += (descs[i].numel + c - 1) / c;
+            return k;
+        });
     P->n_tensors = n_tensors;
     P->n_groups = n_groups;
     P->chunk_elems = chunk_elems;
@@ -1683,18 +1716,19 @@ MGOPT_API int mgopt_grad_norm_noalloc(const void* grads_dev, int32_t grad_dtype,
                                       double max_norm, float* norm_dev, float* coef_dev, float* found_inf_dev,
                                       void* stream) {
     if (n < 1 || grads_dev == nullptr) return fail(MGOPT_E_INVALID, "need n >= 1 and a gradient buffer");
-    const int64_t chunks = (n + kNormChunk - 1) / kNormChunk;
-    if (chunks > kScratchPartials)
+    if (n > kScratchPartials * kNormChunk)
         return fail(MGOPT_E_LIMIT, "n = " + std::to_string(n) + " is above the allocation-free norm's maximum of " +
                                        std::to_string(kScratchPartials * kNormChunk) + " elements");
+    const int64_t chunk = norm_chunk_for([n](int64_t c) { return (n + c - 1) / c; });
+    const int64_t chunks = (n + chunk - 1) / chunk;
     Partial* part = nullptr;
     if (int rc = scratch_on_current_device(&part)) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 grid(static_cast<unsigned>(chunks));
     switch (grad_dtype) {
-        case MGOPT_F32: launch_norm_flat<float>(grads_dev, n, scale_dev, part, grid, s); break;
-        case MGOPT_F16: launch_norm_flat<_Float16>(grads_dev, n, scale_dev, part, grid, s); break;
-        case MGOPT_BF16: launch_norm_flat<Bf16>(grads_dev, n, scale_dev, part, grid, s); break;
+        case MGOPT_F32: launch_norm_flat<float>(grads_dev, n, chunk, scale_dev, part, grid, s); break;
+        case MGOPT_F16: launch_norm_flat<_Float16>(grads_dev, n, chunk, scale_dev, part, grid, s); break;
+        case MGOPT_BF16: launch_norm_flat<Bf16>(grads_dev, n, chunk, scale_dev, part, grid, s); break;
         default: return fail(MGOPT_E_INVALID, "bad grad dtype");
     }
     if (int rc = launch_check("norm_flat_kernel")) return rc;
