@@ -70,15 +70,21 @@ constexpr bool kNtStore = true;      // nontemporal stores of param/exp_avg/exp_
 // against 2.31).
 constexpr int kNormUnroll = 4;
 constexpr int kNormVec16 = 4;
-// Pass 2 reads the gradients pass 1 has just read.  When a plan's gradients
-// fit in the MI355X's 256 MB Infinity Cache (the memory-side cache in front
-// of HBM), pass 1 reads them with ordinary loads, which allocate there, and
-// pass 2's gradient reads hit it.  Measured on GPT-2-small (249 MB of fp16
-// gradients): pass 2 0.513 ms against 0.560 ms after nontemporal pass-1
-// loads, the whole step 0.573 against 0.614 ms.  Larger sets keep
-// nontemporal pass-1 loads: allocating made pass 1 up to 15 % slower on the
-// 2.6 GB and 16 GB gradient sets, with no gain in pass 2 beyond run-to-run
-// spread.  Nontemporal pass-2 gradient loads still hit the cache.
+// Pass 2 reads the gradients pass 1 has just read.  Pass 1 reads the last
+// kCachedGradBytes of them with ordinary loads, which allocate in the MI355X's
+// 256 MB Infinity Cache (the memory-side cache in front of HBM), and all
+// before them with nontemporal loads, which do not; pass 2 then starts with
+// the chunks whose gradients are there (its nontemporal loads hit them).
+// Those loads also push the previous pass 2's last writes out of the cache
+// while pass 1 leaves HBM's write side idle, so the new pass 2's first writes
+// find room.  Whole step, measured in one process on the same buffers, at 0 /
+// 64 / 128 / 192 / 224 / 256 / 320 / 600 MiB: GPT-2-small, 249 MB of fp16
+// gradients, 598 / 590 / 584 / 569 / 556 / 550 / 551 / 551 us; its fp32
+// gradients (498 MB) written back 804 / 797 / 791 / 771 / 764 / 749 / 761 / 780;
+// GPT-1.3B bf16 (2.6 GB) 6.263 / 6.242 / 6.243 / 6.246 / 6.230 / 6.174 / 6.159 /
+// 6.166 ms; 2.8e9 bf16 of the Qwen3-8B shapes 12.77 / 12.77 / 12.71 / 12.71 /
+// 12.69 / 12.68 / 12.68 / 12.72; 20,000 ragged tensors (5 GB of fp16) within
+// their run-to-run 1 % up to 256 MiB and 2 % slower at 600.
 constexpr int64_t kCachedGradBytes = int64_t(256) << 20;
 // pass 1 has its own chunk table, whatever the pass-2 chunk size: at most
 // kNormChunk elements per chunk and work-group, so that the finalize kernel
@@ -377,6 +383,7 @@ struct NormArgs {
     uint32_t chunk_begin;
     uint32_t count;         // chunks of this launch's class
     uint32_t partial_base;  // first partial slot of this launch
+    uint32_t cached_from;   // chunks of this launch from here on are read into the Infinity Cache
     // folded form only: the ticket counter, the plan's partial count and the finalize outputs
     uint32_t* ticket;
     uint32_t total;
@@ -572,9 +579,8 @@ __device__ __forceinline__ void reset_ticket(uint32_t* ticket) {
 // pass 1: unscale + non-finite flag + sum of squares
 // ---------------------------------------------------------------------------
 
-// NT: nontemporal gradient loads (sets larger than the Infinity Cache).
 // FOLD: small plans; the last work-group also runs the finalize.
-template <typename GT, bool NT, bool FOLD>
+template <typename GT, bool FOLD>
 __global__ void __launch_bounds__(kBlock) norm_kernel(const NormArgs a) {
     // work-group slot r (XCD-remapped) sums pass-1 chunk r of its class into
     // partial r: the partials' order does not depend on the remapping
@@ -586,8 +592,11 @@ __global__ void __launch_bounds__(kBlock) norm_kernel(const NormArgs a) {
     if (g != nullptr) {
         const int64_t numel = a.tensors[ck.tensor].numel;
         const int64_t start = static_cast<int64_t>(ck.index) * a.chunk_elems;
-        norm_chunk<GT, NT>(g + start, min(a.chunk_elems, numel - start), inv_scale_of(a.scale), a.scale != nullptr, acc,
-                           bad);
+        const int64_t len = min(a.chunk_elems, numel - start);
+        if (FOLD || slot >= a.cached_from)
+            norm_chunk<GT, false>(g + start, len, inv_scale_of(a.scale), a.scale != nullptr, acc, bad);
+        else
+            norm_chunk<GT, true>(g + start, len, inv_scale_of(a.scale), a.scale != nullptr, acc, bad);
     }
     block_reduce<kBlock>(acc, bad);
     if constexpr (!FOLD) {
@@ -762,6 +771,7 @@ struct AdamArgs {
     const TensorConst* consts;
     int64_t chunk_elems;
     uint32_t chunk_begin;
+    uint32_t first;  // the launch's last `first` chunks go first (a multiple of kXcds)
     int32_t writeback;
 };
 
@@ -974,8 +984,10 @@ __device__ __forceinline__ void adamw_chunk(const AdamArgs& a, const Chunk ck, G
 
 template <typename GT, int LOWP>
 __global__ void __launch_bounds__(kAdamBlock) adamw_kernel(const AdamArgs a) {
-    const uint32_t cidx = a.chunk_begin + xcd_item<kXcdMapAdam>(blockIdx.x, gridDim.x);
-    const Chunk ck = a.chunks[cidx];
+    const uint32_t rest = gridDim.x - a.first;
+    const uint32_t item = blockIdx.x < a.first ? rest + xcd_item<kXcdMapAdam>(blockIdx.x, a.first)
+                                               : xcd_item<kXcdMapAdam>(blockIdx.x - a.first, rest);
+    const Chunk ck = a.chunks[a.chunk_begin + item];
     const TensorConst k = a.consts[ck.tensor];
     if (k.flags & kcSkip) return;  // a skipped step, or no gradient this step
     adamw_chunk<GT, LOWP>(a, ck, static_cast<GT*>(a.grads[ck.tensor]), k);
@@ -1218,6 +1230,8 @@ struct mgopt_plan {
         uint32_t norm_begin;    // first entry of the class in the pass-1 chunk table
         uint32_t norm_count;    // pass-1 chunks (= work-groups = partials) of the class
         uint32_t partial_base;  // first partial slot of the class
+        uint32_t cached_from;   // pass-1 chunks of the class from here on leave their gradients in the Infinity Cache
+        uint32_t first;         // pass 2 starts with this many of the class's last chunks, whose gradients are there
     };
     int64_t n_partials = 0;
     int64_t grad_bytes = 0;  // all gradients of the plan, for pass 1's load policy
@@ -1249,15 +1263,14 @@ int launch_norm(const mgopt_plan* P, const mgopt_plan::Class& c, const float* sc
     // class's partials exactly as one launch would
     for (uint64_t done = 0; done < c.norm_count; done += kMaxGroupsPerLaunch) {
         const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(c.norm_count - done, kMaxGroupsPerLaunch));
+        const uint32_t cached = static_cast<uint32_t>(std::max<uint64_t>(c.cached_from, done) - done);
         NormArgs a{P->d_tensors, P->d_norm_chunks, P->d_grads, P->d_partials, scale, P->norm_chunk,
-                   static_cast<uint32_t>(c.norm_begin + done), n, static_cast<uint32_t>(c.partial_base + done),
+                   static_cast<uint32_t>(c.norm_begin + done), n, static_cast<uint32_t>(c.partial_base + done), cached,
                    P->d_tickets, static_cast<uint32_t>(P->n_partials), fin};
         if (P->fold)
-            hipLaunchKernelGGL((norm_kernel<GT, false, true>), dim3(n), dim3(kBlock), 0, s, a);
-        else if (P->grad_bytes <= kCachedGradBytes)
-            hipLaunchKernelGGL((norm_kernel<GT, false, false>), dim3(n), dim3(kBlock), 0, s, a);
+            hipLaunchKernelGGL((norm_kernel<GT, true>), dim3(n), dim3(kBlock), 0, s, a);
         else
-            hipLaunchKernelGGL((norm_kernel<GT, true, false>), dim3(n), dim3(kBlock), 0, s, a);
+            hipLaunchKernelGGL((norm_kernel<GT, false>), dim3(n), dim3(kBlock), 0, s, a);
         if (int rc = launch_check("norm_kernel")) return rc;
     }
     return 0;
@@ -1471,6 +1484,30 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
         }
     }
     P->n_chunks = static_cast<int64_t>(chunks.size());
+    int64_t cacheable = kCachedGradBytes;  // bytes of the cache not yet spoken for
+    for (auto& c : P->classes) {
+        c.cached_from = c.norm_count;
+        c.first = 0;
+        // a larger set: its last gradients, for a pass 2 of one launch; without
+        // a pass 2 (clip_grad_norm_ over parameters of another optimizer) none
+        if (P->grad_bytes > kCachedGradBytes && (!with_state || P->classes.size() > 1 || c.count > kMaxGroupsPerLaunch))
+            continue;
+        const int64_t size = dtype_size(c.grad_dtype);
+        while (c.cached_from > 0) {
+            const Chunk& k = norm_chunks[c.norm_begin + c.cached_from - 1];
+            const int64_t start = static_cast<int64_t>(k.index) * P->norm_chunk;
+            const int64_t len = std::min(P->norm_chunk, descs[k.tensor].numel - start);
+            if (len * size > cacheable) break;
+            cacheable -= len * size;
+            // the pass-2 chunks that start inside this one
+            c.first += static_cast<uint32_t>((start + len + chunk_elems - 1) / chunk_elems -
+                                             (start + chunk_elems - 1) / chunk_elems);
+            --c.cached_from;
+        }
+        // whole gradient sets that fit need no order; otherwise whole rounds of
+        // the XCDs, so that a work-group's XCD stays blockIdx % kXcds
+        c.first = c.cached_from == 0 ? 0 : c.first / kXcds * kXcds;
+    }
 
     auto cleanup = [&](int rc) {
         mgopt_plan_destroy(P);
@@ -1618,10 +1655,11 @@ MGOPT_API int mgopt_adamw_step(mgopt_plan* P, const mgopt_group_hparams* groups,
         if (int rc = launch_check("prologue_kernel")) return rc;
     }
 
-    AdamArgs a{P->d_tensors, P->d_chunks, P->d_grads, P->d_consts, P->chunk_elems, 0,
+    AdamArgs a{P->d_tensors, P->d_chunks, P->d_grads, P->d_consts, P->chunk_elems, 0, 0,
                (flags & MGOPT_WRITEBACK_GRADS) ? 1 : 0};
     for (const auto& c : P->classes) {
         a.chunk_begin = c.begin;
+        a.first = c.first;
         int rc = 0;
         switch (c.grad_dtype) {
             case MGOPT_F32: rc = launch_adamw_lowp<float>(a, c.lowp_dtype, c.count, f, s); break;
