@@ -891,7 +891,10 @@ struct Group {
                 Vec4<GT> go;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) go.e[j] = GradIO<GT>::from_f32(gc[4 * k + j]);
-                store4(G + e + 4 * k, go);
+                if constexpr (sizeof(GT) == 4)
+                    st16<kNtStore>(reinterpret_cast<float*>(G) + e + 4 * k, __builtin_bit_cast(f32x4, go));
+                else
+                    st8<kNtStore>(G + e + 4 * k, __builtin_bit_cast(u32x2, go));
             }
         }
     }
