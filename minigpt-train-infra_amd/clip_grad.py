@@ -26,6 +26,12 @@ _GRAD_PLANS: dict[tuple, tuple[int, list[int]]] = {}
 _last_fast: tuple[tuple, weakref.ref] | None = None   # (id tuple, engine) of the last fused-path call
 
 
+def _clip_chunk(grads: list[torch.Tensor]) -> int:
+    """Elements per work-group of the in-place scaling: 4 KB of gradients
+    (mgopt.hip, scale_grads_kernel)."""
+    return 4096 // max(g.element_size() for g in grads)
+
+
 def _norm_only(grads: list[torch.Tensor], max_norm: float, error_if_nonfinite: bool) -> torch.Tensor:
     dev = grads[0].device
     if dev.type != "cuda":
@@ -47,7 +53,8 @@ def _norm_only(grads: list[torch.Tensor], max_norm: float, error_if_nonfinite: b
             descs[i].lowp_dtype = N.NONE
         plan = ctypes.c_void_p()
         with torch.cuda.device(dev):
-            N.check(lib.mgopt_plan_create(descs, len(grads), 1, None, 65536, ctypes.byref(plan)), "mgopt_plan_create")
+            N.check(lib.mgopt_plan_create(descs, len(grads), 1, None, _clip_chunk(grads), ctypes.byref(plan)),
+                    "mgopt_plan_create")
         if len(_GRAD_PLANS) > 16:
             old_key = next(iter(_GRAD_PLANS))
             lib.mgopt_plan_destroy(ctypes.c_void_p(_GRAD_PLANS.pop(old_key)[0]))

@@ -105,6 +105,16 @@ constexpr int64_t kCachedGradBytes = int64_t(256) << 20;
 constexpr int64_t kNormChunk = 131072;
 constexpr int64_t kNormChunkMin = 16384;
 constexpr int64_t kNormGroups = 2048;
+// Without a pass 2, clip_grad_norm_'s second pass reads and rewrites every
+// gradient, and what it writes takes the cache's lines too: pass 1 leaves sets
+// of at most kClipCachedBytes there, larger ones not at all, and the scaling
+// uses ordinary accesses up to kScaleCachedBytes.  Both passes, cached against
+// nontemporal pass 1: 78 MB 35.4 (ordinary scaling) / 37.3 (nontemporal)
+// against 37.1 / 39.6 us, 128 MB 69.6 / 60.0 against 65.8 / 63.1, 170 MB 94.8 /
+// 79.6 against 88.0 / 82.6, 249 MB 135.2 / 130.5 against 122.5 / 118.4, 498 MB
+// with the last 256 MB cached 264 / 246 against 239 / 235.
+constexpr int64_t kClipCachedBytes = int64_t(192) << 20;
+constexpr int64_t kScaleCachedBytes = int64_t(96) << 20;
 // Small plans run a step as three kernels instead of five: pass 1 with the
 // finalize in its last work-group, pass 2 with the prologue folded in, and
 // the scaler update.  A plan qualifies with at most kFoldElems elements, no
@@ -1101,7 +1111,14 @@ __global__ void scaler_kernel(float* scale, int32_t* tracker, FoundList fl, int3
 // grad scaling for the stand-alone clip path, master sync, synthetic data
 // ---------------------------------------------------------------------------
 
-template <typename GT>
+// g = g * coef in place, the second pass of a clip without an optimizer step.
+// Bound by HBM reads and writes.  As in pass 2, a 4-KB chunk in 16-B accesses
+// on half of a work-group's lanes keeps work-groups short: both passes of the
+// clip over 249 MB of bf16 took 118 us with 4-KB chunks, 127 with 8-KB, 132
+// with 16-KB and 139 with 128-KB ones; 8-B accesses 137, 256-thread
+// work-groups 124 (2.6 GB: 1.18 / 1.28 / 1.33 / 1.36 / 1.36 / 1.24 ms).
+// NT: nontemporal accesses, for sets above kScaleCachedBytes.
+template <typename GT, bool NT>
 __global__ void __launch_bounds__(kBlock)
     scale_grads_kernel(const DevTensor* tensors, const Chunk* chunks, void* const* grads, const float* coefp,
                        int64_t chunk_elems, uint32_t chunk_begin) {
@@ -1112,9 +1129,23 @@ __global__ void __launch_bounds__(kBlock)
     const int64_t start = static_cast<int64_t>(ck.index) * chunk_elems;
     const int64_t len = min(chunk_elems, tensors[ck.tensor].numel - start);
     g += start;
+    constexpr int W = 16 / sizeof(GT);
     int64_t done = 0;
-    if (aligned(g, sizeof(GT) * 4)) {
-        // four elements per thread per access, as torch's vectorised _foreach_mul_ reads them
+    if (aligned(g, 16)) {
+        const int64_t nvec = len / W;
+        for (int64_t i = threadIdx.x; i < nvec; i += kBlock) {
+            float* at = reinterpret_cast<float*>(g + W * i);
+            GT e[W];
+            const f32x4 x = ld16<NT>(at);
+            std::memcpy(e, &x, 16);
+#pragma unroll
+            for (int k = 0; k < W; ++k) e[k] = GradIO<GT>::from_f32(GradIO<GT>::to_f32(e[k]) * coef);
+            f32x4 y;
+            std::memcpy(&y, e, 16);
+            st16<NT>(at, y);
+        }
+        done = nvec * W;
+    } else if (aligned(g, sizeof(GT) * 4)) {
         const int64_t nvec = len / 4;
         for (int64_t i = threadIdx.x; i < nvec; i += kBlock) {
             Vec4<GT> q = load4(g + 4 * i);
@@ -1355,6 +1386,16 @@ int launch_adamw_lowp(const AdamArgs& a, int32_t lowp, uint32_t count, const Fol
     }
 }
 
+template <typename GT>
+void launch_scale(const mgopt_plan* P, const float* coef, uint32_t n, uint32_t begin, hipStream_t s) {
+    if (P->grad_bytes > kScaleCachedBytes)
+        hipLaunchKernelGGL((scale_grads_kernel<GT, true>), dim3(n), dim3(kBlock), 0, s, P->d_tensors, P->d_chunks,
+                           P->d_grads, coef, P->chunk_elems, begin);
+    else
+        hipLaunchKernelGGL((scale_grads_kernel<GT, false>), dim3(n), dim3(kBlock), 0, s, P->d_tensors, P->d_chunks,
+                           P->d_grads, coef, P->chunk_elems, begin);
+}
+
 int dtype_size(int32_t dt) {
     switch (dt) {
         case MGOPT_F32: return 4;
@@ -1510,13 +1551,13 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
         if (c.count) P->classes.push_back(c);
     }
     P->n_chunks = static_cast<int64_t>(n_chunks);
-    int64_t cacheable = kCachedGradBytes;  // bytes of the cache not yet spoken for
+    const int64_t cache_limit = with_state ? kCachedGradBytes : kClipCachedBytes;
+    int64_t cacheable = cache_limit;  // bytes of the cache not yet spoken for
     for (auto& c : P->classes) {
         c.cached_from = c.norm_count;
         c.first = 0;
-        // a larger set: its last gradients, for a pass 2 of one launch; without
-        // a pass 2 (clip_grad_norm_ over parameters of another optimizer) none
-        if (P->grad_bytes > kCachedGradBytes && (!with_state || P->classes.size() > 1 || c.count > kMaxGroupsPerLaunch))
+        // a larger set: its last gradients, for a pass 2 of one launch
+        if (P->grad_bytes > cache_limit && (!with_state || P->classes.size() > 1 || c.count > kMaxGroupsPerLaunch))
             continue;
         const int64_t size = dtype_size(c.grad_dtype);
         auto span = std::upper_bound(norm_spans.begin(), norm_spans.end(), c.norm_begin + c.norm_count - 1,
@@ -1735,19 +1776,11 @@ MGOPT_API int mgopt_scale_grads(mgopt_plan* P, const float* coef_dev, void* stre
     for (const auto& c : P->classes) {
         for (uint64_t done = 0; done < c.count; done += kMaxGroupsPerLaunch) {
             const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(c.count - done, kMaxGroupsPerLaunch));
+            const uint32_t begin = static_cast<uint32_t>(c.begin + done);
             switch (c.grad_dtype) {
-                case MGOPT_F32:
-                    hipLaunchKernelGGL(scale_grads_kernel<float>, dim3(n), dim3(kBlock), 0, s, P->d_tensors, P->d_chunks,
-                                       P->d_grads, coef_dev, P->chunk_elems, static_cast<uint32_t>(c.begin + done));
-                    break;
-                case MGOPT_F16:
-                    hipLaunchKernelGGL(scale_grads_kernel<_Float16>, dim3(n), dim3(kBlock), 0, s, P->d_tensors,
-                                       P->d_chunks, P->d_grads, coef_dev, P->chunk_elems, static_cast<uint32_t>(c.begin + done));
-                    break;
-                case MGOPT_BF16:
-                    hipLaunchKernelGGL(scale_grads_kernel<Bf16>, dim3(n), dim3(kBlock), 0, s, P->d_tensors, P->d_chunks,
-                                       P->d_grads, coef_dev, P->chunk_elems, static_cast<uint32_t>(c.begin + done));
-                    break;
+                case MGOPT_F32: launch_scale<float>(P, coef_dev, n, begin, s); break;
+                case MGOPT_F16: launch_scale<_Float16>(P, coef_dev, n, begin, s); break;
+                case MGOPT_BF16: launch_scale<Bf16>(P, coef_dev, n, begin, s); break;
                 default: return fail(MGOPT_E_INVALID, "bad grad dtype");
             }
             if (int rc = launch_check("scale_grads_kernel")) return rc;
