@@ -109,7 +109,7 @@ typedef struct mgopt_plan mgopt_plan;
  * dispatch torch builds per call in torch/optim/adam.py:139-212 _init_group
  * and in _foreach_norm's tensor lists, clip_grad.py:85-96): pass 2 (the AdamW
  * update) works in chunks of chunk_elems elements, which must be a positive
- * multiple of 512; pass 1 (the norm) in chunks of 131,072.  steps_dev is a
+ * multiple of 512; pass 1 (the norm) in chunks of its own.  steps_dev is a
  * caller-owned float[n_tensors] holding each tensor's AdamW step count
  * (torch/optim/adam.py:168-176 state["step"]). */
 MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensors, int32_t n_groups,
@@ -176,6 +176,14 @@ MGOPT_API int mgopt_grad_norm(mgopt_plan* plan, const float* scale_dev, double m
 MGOPT_API int mgopt_adamw_step(mgopt_plan* plan, const mgopt_group_hparams* groups, const double* bc_dev,
                                int64_t bc_cap, const float* scale_dev, const float* coef_dev,
                                const float* found_inf_dev, int32_t flags, void* stream);
+
+/* Writes n_groups hyper-parameter sets to dst_dev (8-byte aligned, on GPU
+ * `device`), the array that a step with MGOPT_GROUPS_ON_DEVICE reads, in stream
+ * order: replays enqueued before it on `stream` still read the earlier
+ * records.  `groups` is read before the call returns.  No reference
+ * counterpart. */
+MGOPT_API int mgopt_write_groups(int32_t device, const mgopt_group_hparams* groups, int32_t n_groups, void* dst_dev,
+                                 void* stream);
 
 /* torch._amp_update_scale_ (torch/amp/grad_scaler.py:469-539, call at 529-536),
  * summing n_found found_inf scalars first as grad_scaler.py:517-527 does. */

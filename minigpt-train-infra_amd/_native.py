@@ -27,6 +27,7 @@ EXPORTS = (
     "mgopt_plan_set_grads",
     "mgopt_grad_norm",
     "mgopt_adamw_step",
+    "mgopt_write_groups",
     "mgopt_scaler_update",
     "mgopt_scale_grads",
     "mgopt_sync_master",
@@ -86,6 +87,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "mgopt_plan_set_grads": (ctypes.c_int, [vp, ctypes.POINTER(vp), vp]),
         "mgopt_grad_norm": (ctypes.c_int, [vp, vp, dbl, vp, vp, vp, vp]),
         "mgopt_adamw_step": (ctypes.c_int, [vp, vp, vp, i64, vp, vp, vp, i32, vp]),
+        "mgopt_write_groups": (ctypes.c_int, [i32, vp, i32, vp, vp]),
         "mgopt_scaler_update": (ctypes.c_int, [vp, vp, ctypes.POINTER(vp), i32, dbl, dbl, i32, vp]),
         "mgopt_scale_grads": (ctypes.c_int, [vp, vp, vp]),
         "mgopt_sync_master": (ctypes.c_int, [vp, vp]),

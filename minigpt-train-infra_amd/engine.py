@@ -39,7 +39,6 @@ FOLD_ELEMS = 1 << 21                # the library's three-kernel limits: at most
 FOLD_TENSOR_CHUNKS = 256            # no tensor of more pass-2 chunks than this, no empty tensor
 BC_INITIAL_CAP = 1024               # first bias-correction table size (steps)
 CAPTURE_BC_CAP = 1 << 16            # fixed table size of a capturable engine (graph replays cannot grow it)
-HP_SLOTS = 4                        # pinned host buffers for device hyper-parameter uploads
 
 
 ROW_MAX = 16384                     # longest row (elements) laid out with its master / m / v rows side by side
@@ -244,9 +243,6 @@ class _Engine:
         if capturable:
             with torch.cuda.device(dev):
                 self.hp_dev = torch.zeros(N.MAX_GROUPS * ctypes.sizeof(N.GroupHparams), dtype=torch.uint8, device=dev)
-            self.hp_slots = [torch.empty(self.hp_dev.numel(), dtype=torch.uint8, pin_memory=True) for _ in range(HP_SLOTS)]
-            self.hp_events: list[torch.cuda.Event | None] = [None] * HP_SLOTS
-            self.hp_slot = 0
         self.reset_iteration()
 
     @property
@@ -588,23 +584,12 @@ class _Engine:
         self.hp_raw = None if any(isinstance(r[0], torch.Tensor) for r in raw) else raw
 
     def upload_hparams(self) -> None:
-        """Copies the group records into the device buffer a capturable
-        engine's kernels read (asynchronous, from a pinned slot, on the
-        current stream)."""
+        """Writes the group records into the device buffer a capturable
+        engine's kernels read (asynchronous, on the current stream)."""
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("hyper-parameters cannot be uploaded during graph capture")
-        k = self.hp_slot
-        if self.hp_events[k] is not None:
-            self.hp_events[k].synchronize()     # the slot may still feed an earlier copy
-        data = np.frombuffer(bytes(self.hp), np.uint8)
-        slot = self.hp_slots[k]
-        slot.numpy()[: data.size] = data
-        with torch.cuda.device(self.device):
-            self.hp_dev[: data.size].copy_(slot[: data.size], non_blocking=True)
-            ev = torch.cuda.Event()
-            ev.record()
-        self.hp_events[k] = ev
-        self.hp_slot = (k + 1) % HP_SLOTS
+        N.check(N.lib().mgopt_write_groups(self.device.index, self.hp_addr, len(self.hp), self.hp_dev.data_ptr(),
+                                           self._stream()), "mgopt_write_groups")
         self.hp_dev_key = self.hp_key
 
     def refresh_hparams(self) -> None:
