@@ -12,6 +12,7 @@ torch/nn/utils/clip_grad.py:120-182 does.
 from __future__ import annotations
 
 import ctypes
+import struct
 import types
 import warnings
 import weakref
@@ -20,19 +21,17 @@ from typing import Iterable
 import torch
 
 from . import _native as N
-from .adamw import engine_of
+from .adamw import _OWNER, engine_of
 
-_GRAD_PLANS: dict[tuple, tuple[int, list[int]]] = {}
+#: plans of gradient sets no engine owns, by the set's key: the device index, then each gradient's length (8 bytes)
+#: and dtype code (1 byte)
+_GRAD_PLANS: dict[bytes, int] = {}
 _last_fast: tuple[tuple, weakref.ref] | None = None   # (id tuple, engine) of the last fused-path call
 
 
-def _clip_chunk(grads: list[torch.Tensor]) -> int:
-    """Elements per work-group of the in-place scaling: 4 KB of gradients
-    (mgopt.hip, scale_grads_kernel)."""
-    return 4096 // max(g.element_size() for g in grads)
-
-
-def _norm_only(grads: list[torch.Tensor], max_norm: float, error_if_nonfinite: bool) -> torch.Tensor:
+def _grad_table(grads: list[torch.Tensor]) -> tuple[bytes, bytes, int]:
+    """What the host helper's clip_table returns, for gradients it leaves to
+    Python: the checks here name what is wrong with them."""
     dev = grads[0].device
     if dev.type != "cuda":
         raise RuntimeError("clip_grad_norm_ runs on the GPU only; there is no CPU path")
@@ -41,39 +40,47 @@ def _norm_only(grads: list[torch.Tensor], max_norm: float, error_if_nonfinite: b
             raise RuntimeError("clip_grad_norm_ needs all gradients on one GPU")
         if not g.is_contiguous():
             raise RuntimeError("clip_grad_norm_ needs contiguous gradients")
+    key = struct.pack("<q", dev.index) + b"".join(struct.pack("<qb", g.numel(), N.dtype_code(g.dtype)) for g in grads)
+    return key, struct.pack(f"<{len(grads)}Q", *(g.data_ptr() for g in grads)), dev.index
+
+
+def _grad_plan(key: bytes) -> int:
+    """A new plan for the gradient set of `key`; the oldest of more than 17 is given back."""
     lib = N.lib()
-    key = (dev.index, tuple((N.dtype_code(g.dtype), g.numel()) for g in grads))
-    entry = _GRAD_PLANS.get(key)
-    if entry is None:
-        descs = (N.TensorDesc * len(grads))()
-        for i, g in enumerate(grads):
-            descs[i].numel = g.numel()
-            descs[i].group = 0
-            descs[i].grad_dtype = N.dtype_code(g.dtype)
-            descs[i].lowp_dtype = N.NONE
-        plan = ctypes.c_void_p()
-        with torch.cuda.device(dev):
-            N.check(lib.mgopt_plan_create(descs, len(grads), 1, None, _clip_chunk(grads), ctypes.byref(plan)),
-                    "mgopt_plan_create")
-        if len(_GRAD_PLANS) > 16:
-            old_key = next(iter(_GRAD_PLANS))
-            lib.mgopt_plan_destroy(ctypes.c_void_p(_GRAD_PLANS.pop(old_key)[0]))
-        entry = (plan.value, [])
-        _GRAD_PLANS[key] = entry
-    plan = ctypes.c_void_p(entry[0])
-    stream = ctypes.c_void_p(N.stream_handle(dev))
-    arr = (ctypes.c_void_p * len(grads))(*[g.data_ptr() for g in grads])
-    N.check(lib.mgopt_plan_set_grads(plan, arr, stream), "mgopt_plan_set_grads")
-    norm = torch.empty((), dtype=torch.float32, device=dev)
-    coef = torch.empty((), dtype=torch.float32, device=dev)
-    N.check(
-        lib.mgopt_grad_norm(plan, None, ctypes.c_double(max_norm), ctypes.c_void_p(norm.data_ptr()),
-                            ctypes.c_void_p(coef.data_ptr()), None, stream),
-        "mgopt_grad_norm",
-    )
+    index, = struct.unpack_from("<q", key)
+    sets = list(struct.iter_unpack("<qb", key[8:]))
+    descs = (N.TensorDesc * len(sets))()
+    for d, (numel, code) in zip(descs, sets):
+        d.numel = numel
+        d.group = 0
+        d.grad_dtype = code
+        d.lowp_dtype = N.NONE
+    # elements per work-group of the in-place scaling: 4 KB of gradients (mgopt.hip, scale_grads_kernel)
+    chunk = 1024 if any(code == N.F32 for _, code in sets) else 2048
+    plan = ctypes.c_void_p()
+    with torch.cuda.device(index):
+        N.check(lib.mgopt_plan_create(descs, len(sets), 1, None, chunk, ctypes.byref(plan)), "mgopt_plan_create")
+    if len(_GRAD_PLANS) > 16:
+        lib.mgopt_plan_destroy(ctypes.c_void_p(_GRAD_PLANS.pop(next(iter(_GRAD_PLANS)))))
+    _GRAD_PLANS[key] = plan.value
+    return plan.value
+
+
+def _norm_only(table: tuple[bytes, bytes, int], max_norm: float, error_if_nonfinite: bool) -> torch.Tensor:
+    key, ptrs, index = table
+    N.lib()
+    plan = _GRAD_PLANS.get(key)
+    if plan is None:
+        plan = _grad_plan(key)
+    stream = N.stream_handle(index)
     # torch checks finiteness (clip_grad.py:110-116) before it scales (:232)
-    _check_finite(norm, error_if_nonfinite)
-    N.check(lib.mgopt_scale_grads(plan, ctypes.c_void_p(coef.data_ptr()), stream), "mgopt_scale_grads")
+    scale = 0 if error_if_nonfinite else N.entry_address("mgopt_scale_grads")
+    rc, norm, coef = N.host().clip_launch(N.entry_address("mgopt_plan_set_grads"), N.entry_address("mgopt_grad_norm"),
+                                          scale, plan, ptrs, max_norm, index, stream)
+    N.check(rc, "clip_grad_norm_")
+    if error_if_nonfinite:
+        _check_finite(norm, error_if_nonfinite)
+        N.check(N.lib().mgopt_scale_grads(plan, coef.data_ptr(), stream), "mgopt_scale_grads")
     return norm
 
 
@@ -118,7 +125,7 @@ def clip_grad_norm_(
         _check_finite(total, error_if_nonfinite, eng)
         return total
 
-    engines = {id(e): e for p in parameters if (e := engine_of(p)) is not None}
+    engines = {id(e): e for p in parameters if (e := engine_of(p)) is not None} if _OWNER else {}
     if len(engines) == 1:
         eng = next(iter(engines.values()))
         grads = eng.current_grads()
@@ -139,10 +146,13 @@ def clip_grad_norm_(
                 "clip_grad_norm_ on a parameter list that is not exactly an optimizer's parameters "
                 "cannot follow GradScaler.unscale_ of that optimizer"
             )
-    grads = [p.grad for p in parameters if p.grad is not None]
-    if not grads:
-        return torch.tensor(0.0)
-    return _norm_only(grads, max_norm, error_if_nonfinite)
+    table = N.host().clip_table(parameters)
+    if table is None:
+        grads = [p.grad for p in parameters if p.grad is not None]
+        if not grads:
+            return torch.tensor(0.0)
+        table = _grad_table(grads)
+    return _norm_only(table, max_norm, error_if_nonfinite)
 
 
 def _check_finite(total: torch.Tensor, error_if_nonfinite: bool, eng=None) -> None:
