@@ -109,7 +109,7 @@ typedef struct mgopt_plan mgopt_plan;
  * dispatch torch builds per call in torch/optim/adam.py:139-212 _init_group
  * and in _foreach_norm's tensor lists, clip_grad.py:85-96): pass 2 (the AdamW
  * update) works in chunks of chunk_elems elements, which must be a positive
- * multiple of 512; pass 1 (the norm) in chunks of its own.  steps_dev is a
+ * multiple of 512, each split over one or more work-groups; pass 1 (the norm) in chunks of its own.  steps_dev is a
  * caller-owned float[n_tensors] holding each tensor's AdamW step count
  * (torch/optim/adam.py:168-176 state["step"]). */
 MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensors, int32_t n_groups,
@@ -117,7 +117,7 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
 
 MGOPT_API int mgopt_plan_destroy(mgopt_plan* plan);
 
-/* Number of pass-2 chunks of the plan (one work-group each). */
+/* Number of pass-2 chunks of the plan. */
 MGOPT_API int64_t mgopt_plan_num_chunks(const mgopt_plan* plan);
 
 /* 1 when the plan runs a step as three kernels (a plan of at most 2,097,152

@@ -41,15 +41,26 @@
 namespace {
 
 constexpr int kBlock = 512;          // work-group size of pass 1, finalize and the helper kernels
-// Pass 2 runs one short work-group per chunk.  With the default 1024-element
-// chunks a 512-thread work-group gives one 4-element group to lanes 0-255
-// and lanes 256-511 retire at once: half of a CU's wave slots carry memory
-// traffic and work-groups turn over quickly.  Measured on MI355X against
-// 256-thread groups, 2048/4096/16384/65536-element chunks and LDS-reserved
-// caps of 2-5 work-groups per CU, this was the fastest or tied on the
-// 8.2B set and within 2 % of the best on 124M-2.5B sets.
-constexpr int kAdamBlock = 512;      // work-group size of pass 2
-constexpr size_t kAdamLds = 0;       // LDS bytes reserved per pass-2 work-group (0: no cap on work-groups per CU)
+// Pass 2 runs one very short work-group per kSubElems elements: of its two
+// waves the first gives each lane one 4-element group, the second retires at
+// once.  A work-group of two waves takes one of a CU's 16 work-group slots, so
+// 16 waves per CU carry memory traffic, and a slot turns over every KB of each
+// stream.  Whole steps, one process, same buffers, 512 threads over 1,024
+// elements (half of them idle; the form before) / 128 over 256 / 64 over 256 /
+// 192 over 256 / 256 over 256 / 128 over 512 / 256 over 512: GPT 4 x 512 bf16
+// 197 / 191 / 199 / 191 / 191 / 201 / 199 us; GPT-2-small fp16 gradients 552 /
+// 536 / 556 / 536 / 547 / 565 / 556 us, fp32 written back 751 / 736 / 759 / 734 /
+// 730 / 770 / 759 us; GPT-1.3B bf16 6.18 / 6.08 / 6.28 / 6.07 / 6.24 / 6.29 / 6.17
+// ms; 2.5e9 elements in 20,000 ragged tensors 11.13 / 11.10 / 11.12 / 11.09 /
+// 11.33 / 11.16 / 11.09 ms; 2.8e9 of the Qwen3-8B shapes 12.78 / 12.73 / 12.84 /
+// 12.73 / 13.12 / 12.90 / 12.80 ms.  128 elements per work-group ran 3-30 %
+// slower.  What counts is the number of waves in flight: 64-thread work-groups
+// held at 16 (or 14, or 20) per CU by reserved LDS measured the same as 128
+// over 256, at 8 14 % slower, at 10 9 %, at 12 2 %, at 26 2 %.
+constexpr int kAdamBlock = 128;      // work-group size of pass 2
+constexpr int64_t kSubElems = 256;   // elements per work-group of pass 2
+constexpr uint32_t kMaxSubShift = 8; // at most 256 work-groups per entry of the chunk table (a user's longer chunks)
+constexpr int kFoldBlock = 512;      // work-group size of the three-kernel step's pass 2, one per chunk
 constexpr int kVec = 4;              // elements per thread per access: 4 = one 16-B fp32 access per lane;
                                      // 8 (two adjacent 16-B accesses) measured 1.8x slower (32-B lane stride)
 // A changed gradient table of at most this many tensors goes to the GPU as the
@@ -149,10 +160,11 @@ constexpr uint32_t kTicketStride = 32;  // uint32 counters per 128-byte line: on
 // A dispatch packet carries its grid size in work-items as a 32-bit value, so
 // launches over more chunks than fit are issued in pieces, each piece given
 // its first chunk (and first partial slot) as arguments.  8,388,607
-// work-groups of 512 threads are the most one packet holds; at 1024-element
-// chunks one piece covers 8.59e9 elements.
+// work-groups of 512 threads are the most one packet holds; pass 2's four
+// 128-thread work-groups per 1,024-element chunk are as many threads, so one
+// piece covers 8.59e9 elements (max_chunks).
 constexpr uint32_t kMaxGroupsPerLaunch = 0xFFFFFFFFu / 512;
-static_assert(kBlock <= 512 && kAdamBlock <= 512, "kMaxGroupsPerLaunch assumes work-groups of at most 512 threads");
+static_assert(kBlock <= 512 && kFoldBlock <= 512, "kMaxGroupsPerLaunch assumes work-groups of at most 512 threads");
 // The command processor hands work-groups to the 8 XCDs round-robin in
 // blockIdx order.  With the remap each XCD instead walks one contiguous range
 // of chunks, so its L2 and address-translation caches see 1/8 of the address
@@ -788,8 +800,10 @@ struct AdamArgs {
     const TensorConst* consts;
     int64_t chunk_elems;
     uint32_t chunk_begin;
-    uint32_t first;  // the launch's last `first` chunks go first (a multiple of kXcds)
+    uint32_t first;  // the work-groups of the launch's last chunks that go first (a multiple of kXcds)
     int32_t writeback;
+    uint32_t shift;     // 1 << shift work-groups per chunk
+    int64_t sub_elems;  // of sub_elems = chunk_elems >> shift elements each
 };
 
 struct ElemConst {
@@ -937,33 +951,22 @@ __device__ __forceinline__ ElemConst elem_const(const TensorConst& k) {
     return c;
 }
 
-// The update of one pass-2 chunk of a tensor that has a gradient.
+// The update of work-group `sub`'s part of one pass-2 chunk of a tensor that
+// has a gradient (nothing where the tensor ends before that part).
 template <typename GT, int LOWP>
-__device__ __forceinline__ void adamw_chunk(const AdamArgs& a, const Chunk ck, GT* __restrict__ g, const TensorConst& k) {
+__device__ __forceinline__ void adamw_chunk(const AdamArgs& a, const Chunk ck, uint32_t sub, GT* __restrict__ g,
+                                            const TensorConst& k) {
     const DevTensor T = a.tensors[ck.tensor];
-    ElemConst c;
-    c.inv = k.inv;
-    c.coef = k.coef;
-    c.decay = k.decay;
-    c.w1 = k.w1;
-    c.w1m1 = k.w1m1;
-    c.b2 = k.b2;
-    c.w2 = k.w2;
-    c.bc2s = k.bc2s;
-    c.eps = k.eps;
-    c.nss = k.nss;
-    c.unscale = (k.flags & kcUnscale) != 0;
-    c.clip = (k.flags & kcClip) != 0;
-    c.do_decay = (k.flags & kcDecay) != 0;
-    c.small = (k.flags & kcSmall) != 0;
-    c.maximize = (k.flags & kcMaximize) != 0;
+    const ElemConst c = elem_const(k);
 
-    const int64_t start = static_cast<int64_t>(ck.index) * a.chunk_elems;
-    const int64_t len = min(a.chunk_elems, T.numel - start);
+    const int64_t off = static_cast<int64_t>(sub) * a.sub_elems;
+    const int64_t start = static_cast<int64_t>(ck.index) * a.chunk_elems + off;
+    const int64_t len = min(a.sub_elems, T.numel - start);
+    if (len <= 0) return;
     const ChunkPtrs cp = chunk_ptrs(T, ck.index, a.chunk_elems);
-    float* __restrict__ P = cp.p;
-    float* __restrict__ M = cp.m;
-    float* __restrict__ V = cp.v;
+    float* __restrict__ P = cp.p + off;
+    float* __restrict__ M = cp.m + off;
+    float* __restrict__ V = cp.v + off;
     g += start;
     void* L = nullptr;
     if constexpr (LOWP != MGOPT_NONE) L = static_cast<uint16_t*>(T.lowp) + start;
@@ -1007,10 +1010,11 @@ __global__ void __launch_bounds__(kAdamBlock) adamw_kernel(const AdamArgs a) {
     const uint32_t rest = gridDim.x - a.first;
     const uint32_t item = blockIdx.x < a.first ? rest + xcd_item<kXcdMapAdam>(blockIdx.x, a.first)
                                                : xcd_item<kXcdMapAdam>(blockIdx.x - a.first, rest);
-    const Chunk ck = a.chunks[a.chunk_begin + item];
+    const Chunk ck = a.chunks[a.chunk_begin + (item >> a.shift)];
     const TensorConst k = a.consts[ck.tensor];
     if (k.flags & kcSkip) return;  // a skipped step, or no gradient this step
-    adamw_chunk<GT, LOWP>(a, ck, static_cast<GT*>(a.grads[ck.tensor]), k);
+    const uint32_t sub = item & ((1u << a.shift) - 1u);
+    adamw_chunk<GT, LOWP>(a, ck, sub, static_cast<GT*>(a.grads[ck.tensor]), k);
 }
 
 // Pass 2 of a small plan with the prologue folded in.  Every thread issues
@@ -1021,7 +1025,7 @@ __global__ void __launch_bounds__(kAdamBlock) adamw_kernel(const AdamArgs a) {
 // tensor's last ticket (or of its only chunk) advances the count once every
 // work-group of the tensor has read it.
 template <typename GT, int LOWP>
-__global__ void __launch_bounds__(kAdamBlock)
+__global__ void __launch_bounds__(kFoldBlock)
     adamw_fold_kernel(const AdamArgs a, const PrologueArgs pa, uint32_t* tickets) {
     const Chunk ck = a.chunks[a.chunk_begin + blockIdx.x];
     const bool skip = pa.found_inf != nullptr && *pa.found_inf != 0.0f;
@@ -1044,7 +1048,7 @@ __global__ void __launch_bounds__(kAdamBlock)
     if (first) q.load(g, P, M, V, threadIdx.x * kVec);
 
     __shared__ TensorConst kc;
-    constexpr uint32_t kLead = kAdamBlock - 64;  // first lane of the last wave
+    constexpr uint32_t kLead = kFoldBlock - 64;  // first lane of the last wave
     const uint32_t nch = static_cast<uint32_t>((T.numel + a.chunk_elems - 1) / a.chunk_elems);
     uint32_t t = 0;
     float count = 0.0f;
@@ -1058,12 +1062,12 @@ __global__ void __launch_bounds__(kAdamBlock)
         const ElemConst c = elem_const(k);
         const bool wb = a.writeback != 0;
         if (first) q.template finish<LOWP>(g, P, M, V, L, threadIdx.x * kVec, c, wb);
-        for (int64_t i = threadIdx.x + kAdamBlock; i < nvec; i += kAdamBlock) {
+        for (int64_t i = threadIdx.x + kFoldBlock; i < nvec; i += kFoldBlock) {
             Group<GT> r;
             r.load(g, P, M, V, i * kVec);
             r.template finish<LOWP>(g, P, M, V, L, i * kVec, c, wb);
         }
-        for (int64_t i = nvec * kVec + threadIdx.x; i < len; i += kAdamBlock) {
+        for (int64_t i = nvec * kVec + threadIdx.x; i < len; i += kFoldBlock) {
             float p = P[i], m = M[i], v = V[i];
             const float gc = adam_elem(GradIO<GT>::to_f32(g[i]), p, m, v, c);
             P[i] = p;
@@ -1390,6 +1394,20 @@ void launch_norm_flat(const void* grads, int64_t n, int64_t chunk, const float* 
         hipLaunchKernelGGL((norm_flat_kernel<GT, true>), grid, dim3(kBlock), 0, s, g, n, chunk, scale, part);
 }
 
+// How a pass-2 chunk splits over work-groups: in 1 << shift parts of kSubElems
+// elements, where chunk_elems is a power of two of them (longer parts otherwise,
+// and where that would be more than 1 << kMaxSubShift).
+uint32_t sub_shift(int64_t chunk_elems) {
+    uint32_t shift = 0;
+    while (shift < kMaxSubShift && (chunk_elems >> shift) % (2 * kSubElems) == 0) ++shift;
+    return shift;
+}
+
+// Chunks one pass-2 launch covers.
+uint32_t max_chunks(uint32_t shift) {
+    return std::min(kMaxGroupsPerLaunch, (0xFFFFFFFFu / static_cast<uint32_t>(kAdamBlock)) >> shift);
+}
+
 // The extra arguments of a folded pass 2.
 struct FoldLaunch {
     PrologueArgs pa;
@@ -1399,14 +1417,14 @@ struct FoldLaunch {
 template <typename GT, int LOWP>
 int launch_adamw(AdamArgs a, uint32_t count, const FoldLaunch* f, hipStream_t s) {
     if (f != nullptr) {  // small plans: one piece
-        hipLaunchKernelGGL((adamw_fold_kernel<GT, LOWP>), dim3(count), dim3(kAdamBlock), 0, s, a, f->pa, f->tickets);
+        hipLaunchKernelGGL((adamw_fold_kernel<GT, LOWP>), dim3(count), dim3(kFoldBlock), 0, s, a, f->pa, f->tickets);
         return launch_check("adamw_fold_kernel");
     }
-    const uint32_t begin = a.chunk_begin;
-    for (uint64_t done = 0; done < count; done += kMaxGroupsPerLaunch) {
-        const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(count - done, kMaxGroupsPerLaunch));
+    const uint32_t begin = a.chunk_begin, most = max_chunks(a.shift);
+    for (uint64_t done = 0; done < count; done += most) {
+        const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(count - done, most));
         a.chunk_begin = static_cast<uint32_t>(begin + done);
-        hipLaunchKernelGGL((adamw_kernel<GT, LOWP>), dim3(n), dim3(kAdamBlock), kAdamLds, s, a);
+        hipLaunchKernelGGL((adamw_kernel<GT, LOWP>), dim3(n << a.shift), dim3(kAdamBlock), 0, s, a);
         if (int rc = launch_check("adamw_kernel")) return rc;
     }
     return 0;
@@ -1593,7 +1611,7 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
         c.cached_from = c.norm_count;
         c.first = 0;
         // a larger set: its last gradients, for a pass 2 of one launch
-        if (P->grad_bytes > cache_limit && (!with_state || P->classes.size() > 1 || c.count > kMaxGroupsPerLaunch))
+        if (P->grad_bytes > cache_limit && (!with_state || P->classes.size() > 1 || c.count > max_chunks(sub_shift(chunk_elems))))
             continue;
         const int64_t size = dtype_size(c.grad_dtype);
         auto span = std::upper_bound(norm_spans.begin(), norm_spans.end(), c.norm_begin + c.norm_count - 1,
@@ -1780,11 +1798,12 @@ MGOPT_API int mgopt_adamw_step(mgopt_plan* P, const mgopt_group_hparams* groups,
         if (int rc = launch_check("prologue_kernel")) return rc;
     }
 
+    const uint32_t shift = sub_shift(P->chunk_elems);
     AdamArgs a{P->d_tensors, P->d_chunks, P->d_grads, P->d_consts, P->chunk_elems, 0, 0,
-               (flags & MGOPT_WRITEBACK_GRADS) ? 1 : 0};
+               (flags & MGOPT_WRITEBACK_GRADS) ? 1 : 0, shift, P->chunk_elems >> shift};
     for (const auto& c : P->classes) {
         a.chunk_begin = c.begin;
-        a.first = c.first;
+        a.first = c.first << shift;
         int rc = 0;
         switch (c.grad_dtype) {
             case MGOPT_F32: rc = launch_adamw_lowp<float>(a, c.lowp_dtype, c.count, f, s); break;

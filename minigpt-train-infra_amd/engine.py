@@ -31,10 +31,9 @@ import torch
 from . import _native as N
 
 ALIGN_ELEMS = 64                    # 256 B of fp32 per arena segment
-DEFAULT_CHUNK = 1024                # elements per pass-2 work-group (pass 1 has its own 128K-element chunks):
-                                    # 512 threads over 1024 elements retire fast and keep half the waves
-                                    # of a CU streaming; 2-13 % faster than 16384 from 124M to 8.2B params
-SMALL_CHUNK = 2048                  # pass-2 chunk of a plan that runs the three-kernel step (below)
+DEFAULT_CHUNK = 1024                # elements per entry of pass 2's chunk table; pass 2 splits an entry over four
+                                    # work-groups, pass 1 has chunks of its own
+SMALL_CHUNK = 2048                  # the same for a plan that runs the three-kernel step (below), one work-group each
 FOLD_ELEMS = 1 << 21                # the library's three-kernel limits: at most this many elements,
 FOLD_TENSOR_CHUNKS = 256            # no tensor of more pass-2 chunks than this, no empty tensor
 BC_INITIAL_CAP = 1024               # first bias-correction table size (steps)
