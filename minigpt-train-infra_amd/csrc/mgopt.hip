@@ -133,6 +133,8 @@ constexpr int64_t kNormGroups = 2048;
 // with the last 256 MB cached 264 / 246 against 239 / 235.
 constexpr int64_t kClipCachedBytes = int64_t(192) << 20;
 constexpr int64_t kScaleCachedBytes = int64_t(96) << 20;
+constexpr int kScaleBlock = 64;      // work-group size of the in-place scaling
+constexpr int64_t kScaleBytes = 1024; // gradient bytes per work-group
 // Small plans run a step as three kernels instead of five: pass 1 with the
 // finalize in its last work-group, pass 2 with the prologue folded in, and
 // the scaler update.  A plan qualifies with at most kFoldElems elements, no
@@ -1152,28 +1154,33 @@ __global__ void scaler_kernel(float* scale, int32_t* tracker, FoundList fl, int3
 // ---------------------------------------------------------------------------
 
 // g = g * coef in place, the second pass of a clip without an optimizer step.
-// Bound by HBM reads and writes.  As in pass 2, a 4-KB chunk in 16-B accesses
-// on half of a work-group's lanes keeps work-groups short: both passes of the
-// clip over 249 MB of bf16 took 118 us with 4-KB chunks, 127 with 8-KB, 132
-// with 16-KB and 139 with 128-KB ones; 8-B accesses 137, 256-thread
-// work-groups 124 (2.6 GB: 1.18 / 1.28 / 1.33 / 1.36 / 1.36 / 1.24 ms).
+// Bound by HBM reads and writes of one stream, so unlike pass 2 it wants every
+// wave slot: single-wave work-groups over 1 KB, one 16-B access per lane.  Whole
+// call (norm and scaling), one process, 512 threads over 4 KB (half of them
+// idle) / 64 over 1 KB / 128 over 2 KB / 256 over 2 KB (half idle) / 128 over 1
+// KB (half idle): 249 MB of bf16 in 148 tensors 134 / 128.6 / 128.3 / 138 / 151
+// us; fp32 in 50 tensors, 240 MB 121 / 118 / 121 / 122 / 140 us, 360 MB 174 /
+// 170 / 175 / 175 / 204 us, 1 GB 471 / 456 / 471 / 476 / 547 us.  Longer chunks
+// in 512-thread work-groups, 8 KB to 128 KB, took 4-15 % more than 4 KB.
 // NT: nontemporal accesses, for sets above kScaleCachedBytes.
 template <typename GT, bool NT>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kScaleBlock)
     scale_grads_kernel(const DevTensor* tensors, const Chunk* chunks, void* const* grads, const float* coefp,
-                       int64_t chunk_elems, uint32_t chunk_begin) {
-    const Chunk ck = chunks[chunk_begin + blockIdx.x];
+                       int64_t chunk_elems, uint32_t chunk_begin, uint32_t shift) {
+    const Chunk ck = chunks[chunk_begin + (blockIdx.x >> shift)];
     GT* g = static_cast<GT*>(grads[ck.tensor]);
     if (g == nullptr) return;
     const float coef = *coefp;
-    const int64_t start = static_cast<int64_t>(ck.index) * chunk_elems;
-    const int64_t len = min(chunk_elems, tensors[ck.tensor].numel - start);
+    const int64_t part = chunk_elems >> shift, sub = blockIdx.x & ((1u << shift) - 1u);
+    const int64_t start = static_cast<int64_t>(ck.index) * chunk_elems + sub * part;
+    const int64_t len = min(part, tensors[ck.tensor].numel - start);
+    if (len <= 0) return;
     g += start;
     constexpr int W = 16 / sizeof(GT);
     int64_t done = 0;
     if (aligned(g, 16)) {
         const int64_t nvec = len / W;
-        for (int64_t i = threadIdx.x; i < nvec; i += kBlock) {
+        for (int64_t i = threadIdx.x; i < nvec; i += kScaleBlock) {
             float* at = reinterpret_cast<float*>(g + W * i);
             GT e[W];
             const f32x4 x = ld16<NT>(at);
@@ -1187,7 +1194,7 @@ __global__ void __launch_bounds__(kBlock)
         done = nvec * W;
     } else if (aligned(g, sizeof(GT) * 4)) {
         const int64_t nvec = len / 4;
-        for (int64_t i = threadIdx.x; i < nvec; i += kBlock) {
+        for (int64_t i = threadIdx.x; i < nvec; i += kScaleBlock) {
             Vec4<GT> q = load4(g + 4 * i);
 #pragma unroll
             for (int k = 0; k < 4; ++k) q.e[k] = GradIO<GT>::from_f32(GradIO<GT>::to_f32(q.e[k]) * coef);
@@ -1195,7 +1202,7 @@ __global__ void __launch_bounds__(kBlock)
         }
         done = nvec * 4;
     }
-    for (int64_t i = done + threadIdx.x; i < len; i += kBlock) g[i] = GradIO<GT>::from_f32(GradIO<GT>::to_f32(g[i]) * coef);
+    for (int64_t i = done + threadIdx.x; i < len; i += kScaleBlock) g[i] = GradIO<GT>::from_f32(GradIO<GT>::to_f32(g[i]) * coef);
 }
 
 template <typename LT>
@@ -1440,14 +1447,25 @@ int launch_adamw_lowp(const AdamArgs& a, int32_t lowp, uint32_t count, const Fol
     }
 }
 
+// In pieces of at most one dispatch packet's work-items.
 template <typename GT>
-void launch_scale(const mgopt_plan* P, const float* coef, uint32_t n, uint32_t begin, hipStream_t s) {
-    if (P->grad_bytes > kScaleCachedBytes)
-        hipLaunchKernelGGL((scale_grads_kernel<GT, true>), dim3(n), dim3(kBlock), 0, s, P->d_tensors, P->d_chunks,
-                           P->d_grads, coef, P->chunk_elems, begin);
-    else
-        hipLaunchKernelGGL((scale_grads_kernel<GT, false>), dim3(n), dim3(kBlock), 0, s, P->d_tensors, P->d_chunks,
-                           P->d_grads, coef, P->chunk_elems, begin);
+int launch_scale(const mgopt_plan* P, const mgopt_plan::Class& c, const float* coef, hipStream_t s) {
+    uint32_t shift = 0;
+    while (shift < kMaxSubShift && (P->chunk_elems >> shift) * static_cast<int64_t>(sizeof(GT)) % (2 * kScaleBytes) == 0)
+        ++shift;
+    const uint32_t most = std::min(kMaxGroupsPerLaunch, (0xFFFFFFFFu / static_cast<uint32_t>(kScaleBlock)) >> shift);
+    for (uint64_t done = 0; done < c.count; done += most) {
+        const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(c.count - done, most)) << shift;
+        const uint32_t begin = static_cast<uint32_t>(c.begin + done);
+        if (P->grad_bytes > kScaleCachedBytes)
+            hipLaunchKernelGGL((scale_grads_kernel<GT, true>), dim3(n), dim3(kScaleBlock), 0, s, P->d_tensors, P->d_chunks,
+                               P->d_grads, coef, P->chunk_elems, begin, shift);
+        else
+            hipLaunchKernelGGL((scale_grads_kernel<GT, false>), dim3(n), dim3(kScaleBlock), 0, s, P->d_tensors, P->d_chunks,
+                               P->d_grads, coef, P->chunk_elems, begin, shift);
+        if (int rc = launch_check("scale_grads_kernel")) return rc;
+    }
+    return 0;
 }
 
 int dtype_size(int32_t dt) {
@@ -1850,17 +1868,14 @@ MGOPT_API int mgopt_scale_grads(mgopt_plan* P, const float* coef_dev, void* stre
     DeviceGuard guard(P->device);
     hipStream_t s = static_cast<hipStream_t>(stream);
     for (const auto& c : P->classes) {
-        for (uint64_t done = 0; done < c.count; done += kMaxGroupsPerLaunch) {
-            const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(c.count - done, kMaxGroupsPerLaunch));
-            const uint32_t begin = static_cast<uint32_t>(c.begin + done);
-            switch (c.grad_dtype) {
-                case MGOPT_F32: launch_scale<float>(P, coef_dev, n, begin, s); break;
-                case MGOPT_F16: launch_scale<_Float16>(P, coef_dev, n, begin, s); break;
-                case MGOPT_BF16: launch_scale<Bf16>(P, coef_dev, n, begin, s); break;
-                default: return fail(MGOPT_E_INVALID, "bad grad dtype");
-            }
-            if (int rc = launch_check("scale_grads_kernel")) return rc;
+        int rc = 0;
+        switch (c.grad_dtype) {
+            case MGOPT_F32: rc = launch_scale<float>(P, c, coef_dev, s); break;
+            case MGOPT_F16: rc = launch_scale<_Float16>(P, c, coef_dev, s); break;
+            case MGOPT_BF16: rc = launch_scale<Bf16>(P, c, coef_dev, s); break;
+            default: rc = fail(MGOPT_E_INVALID, "bad grad dtype");
         }
+        if (rc) return rc;
     }
     return 0;
 }
