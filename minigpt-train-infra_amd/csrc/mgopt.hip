@@ -41,23 +41,30 @@
 namespace {
 
 constexpr int kBlock = 512;          // work-group size of pass 1, finalize and the helper kernels
-// Pass 2 runs one very short work-group per kSubElems elements: of its two
-// waves the first gives each lane one 4-element group, the second retires at
-// once.  A work-group of two waves takes one of a CU's 16 work-group slots, so
-// 16 waves per CU carry memory traffic, and a slot turns over every KB of each
-// stream.  Whole steps, one process, same buffers, 512 threads over 1,024
-// elements (half of them idle; the form before) / 128 over 256 / 64 over 256 /
-// 192 over 256 / 256 over 256 / 128 over 512 / 256 over 512: GPT 4 x 512 bf16
-// 197 / 191 / 199 / 191 / 191 / 201 / 199 us; GPT-2-small fp16 gradients 552 /
-// 536 / 556 / 536 / 547 / 565 / 556 us, fp32 written back 751 / 736 / 759 / 734 /
-// 730 / 770 / 759 us; GPT-1.3B bf16 6.18 / 6.08 / 6.28 / 6.07 / 6.24 / 6.29 / 6.17
-// ms; 2.5e9 elements in 20,000 ragged tensors 11.13 / 11.10 / 11.12 / 11.09 /
-// 11.33 / 11.16 / 11.09 ms; 2.8e9 of the Qwen3-8B shapes 12.78 / 12.73 / 12.84 /
-// 12.73 / 13.12 / 12.90 / 12.80 ms.  128 elements per work-group ran 3-30 %
-// slower.  What counts is the number of waves in flight: 64-thread work-groups
-// held at 16 (or 14, or 20) per CU by reserved LDS measured the same as 128
-// over 256, at 8 14 % slower, at 10 9 %, at 12 2 %, at 26 2 %.
-constexpr int kAdamBlock = 128;      // work-group size of pass 2
+// Pass 2 runs one very short work-group per kSubElems elements, in dispatch
+// order: work-group b takes the elements from 256 b on, so the eight XCDs walk
+// one window together, a KB of each stream each in turn.  Of a work-group's three
+// waves the first gives each lane one 4-element group and the others retire
+// at once: 32 wave slots a CU let ten work-groups in, and ten to sixteen waves
+// of memory traffic per CU are what HBM takes best.  Whole steps, one process, same
+// buffers, in us (ms from GPT-1.3B on):
+//                                    GPT 4x512  GPT-2-small  fp32, grads  GPT-1.3B  2.5e9 in 20k  2.8e9 Qwen3-
+//   threads, elements, order         bf16       fp16 grads   written back bf16      ragged        8B shapes
+//   512, 1,024, a range per XCD      197        552          751          6.18      11.13         12.78
+//   128, 256, a range per XCD        193        542          737          6.05      11.09         12.67
+//   192, 256, dispatch order (this)  180        528          724          5.77      11.06         12.32
+//   128, 256, dispatch order         184        531          728          5.78      11.07         12.32
+//   64, 256, dispatch order          187        548          750          6.21      11.29         12.90
+//   256, 256, dispatch order         181        541          719          6.31      11.67         13.27
+//   128, 512, dispatch order         190        553          747          7.34      11.58         14.88
+//   256, 512, dispatch order         188        545          734          6.86      11.52         14.66
+//   320, 512, dispatch order         183        548          709          6.16      11.87         13.34
+//   512, 1,024, dispatch order       195        562          751          6.03      11.16         12.90
+// (the first row from another process).  128 elements per work-group ran 3-30 %
+// slower.  64-thread work-groups held at 14 a CU by reserved LDS measured as
+// 192 over 256 do; held at 8, 14 % slower, at 10 9 %, at 26 2 %.  XCDs taking
+// turns by 4 KB up to 4 MB instead of 1 KB: 0-8 % slower.
+constexpr int kAdamBlock = 192;      // work-group size of pass 2
 constexpr int64_t kSubElems = 256;   // elements per work-group of pass 2
 constexpr uint32_t kMaxSubShift = 8; // at most 256 work-groups per entry of the chunk table (a user's longer chunks)
 constexpr int kFoldBlock = 512;      // work-group size of the three-kernel step's pass 2, one per chunk
@@ -162,21 +169,11 @@ constexpr uint32_t kTicketStride = 32;  // uint32 counters per 128-byte line: on
 // A dispatch packet carries its grid size in work-items as a 32-bit value, so
 // launches over more chunks than fit are issued in pieces, each piece given
 // its first chunk (and first partial slot) as arguments.  8,388,607
-// work-groups of 512 threads are the most one packet holds; pass 2's four
-// 128-thread work-groups per 1,024-element chunk are as many threads, so one
-// piece covers 8.59e9 elements (max_chunks).
+// work-groups of 512 threads are the most one packet holds; with pass 2's four
+// 192-thread work-groups per 1,024-element chunk one piece covers 5.7e9
+// elements (max_chunks).
 constexpr uint32_t kMaxGroupsPerLaunch = 0xFFFFFFFFu / 512;
 static_assert(kBlock <= 512 && kFoldBlock <= 512, "kMaxGroupsPerLaunch assumes work-groups of at most 512 threads");
-// The command processor hands work-groups to the 8 XCDs round-robin in
-// blockIdx order.  With the remap each XCD instead walks one contiguous range
-// of chunks, so its L2 and address-translation caches see 1/8 of the address
-// window instead of every eighth chunk of all of it.  Measured on the
-// Qwen3-8B-shaped set: pass 2 0.1-0.2 ms faster (within run-to-run spread),
-// pass 1 0.0-0.3 ms slower, so only pass 2 uses it.
-constexpr bool kXcdMapAdam = true;
-constexpr bool kXcdMapNorm = false;
-constexpr uint32_t kXcds = 8;
-
 struct DevTensor {
     float* param;   // fp32 param or fp32 master
     void* lowp;     // bf16/fp16 model param or nullptr
@@ -316,17 +313,6 @@ __device__ __forceinline__ void store4(T* p, const Vec4<T>& r) {
 }
 
 __device__ __forceinline__ bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
-
-// Work item of work-group `bid` in a grid of `n`: a bijection of [0, n).
-// Work-group bid runs on XCD bid % 8; XCD x gets items
-// [x*per + min(x, rem), ...) of length per + (x < rem), in order.
-template <bool kRemap>
-__device__ __forceinline__ uint32_t xcd_item(uint32_t bid, uint32_t n) {
-    if constexpr (!kRemap) return bid;
-    const uint32_t per = n / kXcds, rem = n % kXcds;
-    const uint32_t x = bid % kXcds;
-    return x * per + min(x, rem) + bid / kXcds;
-}
 
 // Native vector types for 16-byte (4 x fp32) and 8-byte (4 x 16-bit) accesses;
 // the nontemporal forms mark streamed data that no later access reuses.
@@ -613,11 +599,10 @@ __device__ __forceinline__ void reset_ticket(uint32_t* ticket) {
 // FOLD: small plans; the last work-group also runs the finalize.
 template <typename GT, bool FOLD>
 __global__ void __launch_bounds__(kBlock) norm_kernel(const NormArgs a) {
-    // work-group slot r (XCD-remapped) sums pass-1 chunk r of its class into
-    // partial r: the partials' order does not depend on the remapping
+    // work-group r sums pass-1 chunk r of its class into partial r
     double acc = 0.0;
     uint32_t bad = 0;
-    const uint32_t slot = xcd_item<kXcdMapNorm>(blockIdx.x, gridDim.x);
+    const uint32_t slot = blockIdx.x;
     const Chunk ck = a.chunks[a.chunk_begin + slot];
     const GT* __restrict__ g = static_cast<const GT*>(a.grads[ck.tensor]);
     if (g != nullptr) {
@@ -802,7 +787,7 @@ struct AdamArgs {
     const TensorConst* consts;
     int64_t chunk_elems;
     uint32_t chunk_begin;
-    uint32_t first;  // the work-groups of the launch's last chunks that go first (a multiple of kXcds)
+    uint32_t first;  // the launch's last `first` work-group parts go first
     int32_t writeback;
     uint32_t shift;     // 1 << shift work-groups per chunk
     int64_t sub_elems;  // of sub_elems = chunk_elems >> shift elements each
@@ -1010,8 +995,7 @@ __device__ __forceinline__ void adamw_chunk(const AdamArgs& a, const Chunk ck, u
 template <typename GT, int LOWP>
 __global__ void __launch_bounds__(kAdamBlock) adamw_kernel(const AdamArgs a) {
     const uint32_t rest = gridDim.x - a.first;
-    const uint32_t item = blockIdx.x < a.first ? rest + xcd_item<kXcdMapAdam>(blockIdx.x, a.first)
-                                               : xcd_item<kXcdMapAdam>(blockIdx.x - a.first, rest);
+    const uint32_t item = blockIdx.x < a.first ? rest + blockIdx.x : blockIdx.x - a.first;
     const Chunk ck = a.chunks[a.chunk_begin + (item >> a.shift)];
     const TensorConst k = a.consts[ck.tensor];
     if (k.flags & kcSkip) return;  // a skipped step, or no gradient this step
@@ -1427,10 +1411,12 @@ int launch_adamw(AdamArgs a, uint32_t count, const FoldLaunch* f, hipStream_t s)
         hipLaunchKernelGGL((adamw_fold_kernel<GT, LOWP>), dim3(count), dim3(kFoldBlock), 0, s, a, f->pa, f->tickets);
         return launch_check("adamw_fold_kernel");
     }
-    const uint32_t begin = a.chunk_begin, most = max_chunks(a.shift);
-    for (uint64_t done = 0; done < count; done += most) {
-        const uint32_t n = static_cast<uint32_t>(std::min<uint64_t>(count - done, most));
-        a.chunk_begin = static_cast<uint32_t>(begin + done);
+    // the piece with the last chunks first: it is the one whose gradients are cached
+    const uint32_t begin = a.chunk_begin, most = max_chunks(a.shift), first = a.first;
+    for (uint32_t piece = (count + most - 1) / most; piece-- > 0;) {
+        const uint32_t n = std::min(count - piece * most, most);
+        a.chunk_begin = begin + piece * most;
+        a.first = (piece + 1) * static_cast<uint64_t>(most) >= count ? std::min(first, n) << a.shift : 0;
         hipLaunchKernelGGL((adamw_kernel<GT, LOWP>), dim3(n << a.shift), dim3(kAdamBlock), 0, s, a);
         if (int rc = launch_check("adamw_kernel")) return rc;
     }
@@ -1628,9 +1614,8 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
     for (auto& c : P->classes) {
         c.cached_from = c.norm_count;
         c.first = 0;
-        // a larger set: its last gradients, for a pass 2 of one launch
-        if (P->grad_bytes > cache_limit && (!with_state || P->classes.size() > 1 || c.count > max_chunks(sub_shift(chunk_elems))))
-            continue;
+        // a larger set: its last gradients
+        if (P->grad_bytes > cache_limit && (!with_state || P->classes.size() > 1)) continue;
         const int64_t size = dtype_size(c.grad_dtype);
         auto span = std::upper_bound(norm_spans.begin(), norm_spans.end(), c.norm_begin + c.norm_count - 1,
                                      [](uint32_t e, const Span& x) { return e < x.first; });
@@ -1648,9 +1633,7 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
                                              (start + chunk_elems - 1) / chunk_elems);
             --c.cached_from;
         }
-        // whole gradient sets that fit need no order; otherwise whole rounds of
-        // the XCDs, so that a work-group's XCD stays blockIdx % kXcds
-        c.first = c.cached_from == 0 ? 0 : c.first / kXcds * kXcds;
+        if (c.cached_from == 0) c.first = 0;  // all of it: no order finds more
     }
 
     auto cleanup = [&](int rc) {
@@ -1821,7 +1804,7 @@ MGOPT_API int mgopt_adamw_step(mgopt_plan* P, const mgopt_group_hparams* groups,
                (flags & MGOPT_WRITEBACK_GRADS) ? 1 : 0, shift, P->chunk_elems >> shift};
     for (const auto& c : P->classes) {
         a.chunk_begin = c.begin;
-        a.first = c.first << shift;
+        a.first = c.first;
         int rc = 0;
         switch (c.grad_dtype) {
             case MGOPT_F32: rc = launch_adamw_lowp<float>(a, c.lowp_dtype, c.count, f, s); break;
