@@ -102,15 +102,22 @@ constexpr int kNormVec16 = 4;
 // the chunks whose gradients are there (its nontemporal loads hit them).
 // Those loads also push the previous pass 2's last writes out of the cache
 // while pass 1 leaves HBM's write side idle, so the new pass 2's first writes
-// find room.  Whole step, measured in one process on the same buffers, at 0 /
-// 64 / 128 / 192 / 224 / 256 / 320 / 600 MiB: GPT-2-small, 249 MB of fp16
-// gradients, 598 / 590 / 584 / 569 / 556 / 550 / 551 / 551 us; its fp32
-// gradients (498 MB) written back 804 / 797 / 791 / 771 / 764 / 749 / 761 / 780;
-// GPT-1.3B bf16 (2.6 GB) 6.263 / 6.242 / 6.243 / 6.246 / 6.230 / 6.174 / 6.159 /
-// 6.166 ms; 2.8e9 bf16 of the Qwen3-8B shapes 12.77 / 12.77 / 12.71 / 12.71 /
-// 12.69 / 12.68 / 12.68 / 12.72; 20,000 ragged tensors (5 GB of fp16) within
-// their run-to-run 1 % up to 256 MiB and 2 % slower at 600.
+// find room.  A set of at least kLongCacheFrom gradient bytes has twice as much
+// read that way: what comes back from the cache is no more, but less of the
+// previous step is left in it.  Whole step, measured in one process on the same
+// buffers, in us (ms from GPT-1.3B on), by MiB read with ordinary loads:
+//                                        0      128    256    320    384    512    640    1024
+//   GPT-2-small, 249 MB fp16             550    537    523    (all of it)
+//   its fp32 written back, 498 MB        744    746    721    731    744    748    (all of it)
+//   GPT 12x1000 fp32, 0.78 GB            1006          983    976    973    971    977    983
+//   GPT 12x1536 bf16, 0.83 GB            1936          1865   1862   1867   1861   1861   1870
+//   GPT-1.3B bf16, 2.6 GB                5.99   6.01   5.72   5.73   5.73   5.67   5.67   5.68
+//   ragged 20,000 fp16, 5.0 GB           11.4          11.1   11.0   11.1   11.1   11.1   11.1
+//   Qwen3-8B, 8 layers bf16, 5.6 GB      12.68  12.83  12.29  12.29  12.29  12.17  12.17  12.17
+//   Qwen3-8B, 24 layers bf16, 11.7 GB    26.7          26.7   26.6   26.6   25.6   25.6   25.6
 constexpr int64_t kCachedGradBytes = int64_t(256) << 20;
+constexpr int64_t kLongCacheFrom = int64_t(640) << 20;
+constexpr int64_t kLongCachedGradBytes = int64_t(512) << 20;
 // pass 1 has its own chunk table, whatever the pass-2 chunk size: at most
 // kNormChunk elements per chunk and work-group, so that the finalize kernel
 // reads one partial per 128K elements on a large set.  Pass 1 + finalize
@@ -1609,7 +1616,9 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
         if (c.count) P->classes.push_back(c);
     }
     P->n_chunks = static_cast<int64_t>(n_chunks);
-    const int64_t cache_limit = with_state ? kCachedGradBytes : kClipCachedBytes;
+    const int64_t cache_limit = !with_state                       ? kClipCachedBytes
+                                : P->grad_bytes >= kLongCacheFrom ? kLongCachedGradBytes
+                                                                  : kCachedGradBytes;
     int64_t cacheable = cache_limit;  // bytes of the cache not yet spoken for
     for (auto& c : P->classes) {
         c.cached_from = c.norm_count;

@@ -1,7 +1,7 @@
-"""Gradient sets larger than the Infinity Cache: pass 1 leaves the last 256 MiB
-of them there and pass 2 starts with those chunks, then does the rest.  Each
-chunk must be updated exactly once whatever the number of chunks left over by
-the split over the eight XCDs."""
+"""Gradient sets larger than the Infinity Cache: pass 1 reads the last 256 MiB
+of them (512 MiB of a set of at least 640 MiB) with loads that allocate there,
+and pass 2 starts with those chunks, then does the rest.  Each chunk must be
+updated exactly once wherever the split falls."""
 
 from __future__ import annotations
 
@@ -34,7 +34,9 @@ def _params(sizes, dtype, seed):
     ((40_000_000, 40_000_000, 1025, 7), torch.float32),     # on another tensor than the last
     ((67_108_865,), torch.float32),                         # one element more than fits
     ((90_000_001, 30_000_000, 30_000_001), torch.bfloat16),
-], ids=["inside", "between", "one-over", "bf16"])
+    ((100_000_001, 67_772_159, 3), torch.float32),          # 640 MiB less 4 bytes: the last with 256 MiB
+    ((100_000_001, 67_772_159, 4), torch.float32),          # 640 MiB: 512 MiB from here on
+], ids=["inside", "between", "one-over", "bf16", "below-long", "long"])
 def test_every_chunk_is_updated_once(sizes, dtype):
     log(f"case: cached first {sizes} {dtype}")
     whole, single = _params(sizes, dtype, 3), _params(sizes, dtype, 3)
