@@ -216,8 +216,8 @@ MGOPT_API int mgopt_plan_flags(mgopt_plan* plan, int* out);
 
 /* The gradient L2 norm of one contiguous gradient buffer of n elements (a
  * flat gradient arena), with the outputs, scaling and arithmetic of
- * mgopt_grad_norm.  It sums the same 131,072-element chunks in the same order
- * as mgopt_grad_norm on a plan holding that buffer as its one tensor in the
+ * mgopt_grad_norm.  It sums the same chunks (of at most 131,072 elements,
+ * fewer on small buffers) in the same order as mgopt_grad_norm on a plan holding that buffer as its one tensor in the
  * five-kernel form (a plan of more than 2,097,152 elements, or any plan made
  * with MGOPT_FOLD=0 in the environment), and is bit-identical to it there; a
  * plan of at most 2,097,152 elements runs the three-kernel form, whose
