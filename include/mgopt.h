@@ -133,7 +133,9 @@ MGOPT_API int mgopt_plan_folded(const mgopt_plan* plan);
 /* Sets the gradient of every tensor for the coming step from a host array of
  * n_tensors device pointers (NULL = this tensor has no grad this step, as
  * p.grad is None is skipped at torch/optim/adam.py:153 and clip_grad.py:228).
- * Uploads only when the pointers changed since the last call. */
+ * Uploads only when the pointers changed since the last call.  In a stream
+ * capture the pointers are always recorded, and every replay sets them again;
+ * once that happened, calls outside a capture upload theirs every time. */
 MGOPT_API int mgopt_plan_set_grads(mgopt_plan* plan, const void* const* grads_host, void* stream);
 
 /* Pass 1 + finalize: the gradient L2 norm.  Replaces

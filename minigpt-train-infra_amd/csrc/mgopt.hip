@@ -70,14 +70,15 @@ constexpr uint32_t kMaxSubShift = 8; // at most 256 work-groups per entry of the
 constexpr int kFoldBlock = 512;      // work-group size of the three-kernel step's pass 2, one per chunk
 constexpr int kVec = 4;              // elements per thread per access: 4 = one 16-B fp32 access per lane;
                                      // 8 (two adjacent 16-B accesses) measured 1.8x slower (32-B lane stride)
-// A changed gradient table of at most this many tensors goes to the GPU as the
-// arguments of a small kernel (4 KB at most): a launch, where the copy from a
-// pinned buffer was a copy, an event that says when the buffer is free again,
-// and a wait between the copy and pass 1.  Clip of GPT-2-small's 148 bf16
+// A changed gradient table of at most this many tensors (and every captured
+// one, in pieces of as many) goes to the GPU as the arguments of a small kernel
+// (4 KB at most): a launch, where the copy from a pinned buffer was a copy, an
+// event that says when the buffer is free again, and a wait between the copy
+// and pass 1.  Clip of GPT-2-small's 148 bf16
 // gradients in new buffers each time: 134 us per call with the copy,
 // 131 with the kernel.
 constexpr int32_t kArgGrads = 480;
-constexpr int kStagingSlots = 4;     // pinned host buffers for the tables of larger sets
+constexpr int kStagingSlots = 4;     // pinned host buffers for the tables of larger sets, outside a capture
 // pass-2 access tuning (measured on MI355X with the Qwen3-8B-shaped set)
 constexpr int kUnroll = 1;           // 4-element accesses in flight per thread before use
 constexpr bool kNtLoad = true;       // nontemporal loads of grad/param/exp_avg/exp_avg_sq
@@ -1338,6 +1339,7 @@ struct mgopt_plan {
     bool has_state = false;  // false: grads-only plan (norm and grad scaling only)
     std::vector<const void*> cached;
     bool grads_uploaded = false;
+    bool table_captured = false;  // a graph holds a write of d_grads, so any replay may have changed it since `cached`
     void* staging[kStagingSlots] = {};
     hipEvent_t staging_ev[kStagingSlots] = {};
     bool staging_used[kStagingSlots] = {};
@@ -1350,6 +1352,13 @@ int launch_check(const char* what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, what);
     return 0;
+}
+
+bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) == hipSuccess) return status == hipStreamCaptureStatusActive;
+    (void)hipGetLastError();  // the legacy stream while another stream captures: it does not capture itself
+    return false;
 }
 
 template <typename GT>
@@ -1732,14 +1741,25 @@ MGOPT_API int mgopt_plan_folded(const mgopt_plan* P) { return P ? (P->fold ? 1 :
 
 MGOPT_API int mgopt_plan_set_grads(mgopt_plan* P, const void* const* grads_host, void* stream) {
     if (!P || !grads_host) return fail(MGOPT_E_INVALID, "NULL argument");
-    if (P->grads_uploaded && std::memcmp(P->cached.data(), grads_host, sizeof(void*) * P->n_tensors) == 0) return 0;
     DeviceGuard guard(P->device);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (P->n_tensors <= kArgGrads) {
-        GradTable t{};
-        std::memcpy(t.p, grads_host, sizeof(void*) * P->n_tensors);
-        hipLaunchKernelGGL(write_grads_kernel, dim3(1), dim3(kBlock), 0, s, t, P->n_tensors, P->d_grads);
-        if (int rc = launch_check("write_grads_kernel")) return rc;
+    const bool capturing = is_capturing(s);
+    if (!capturing && !P->table_captured && P->grads_uploaded &&
+        std::memcmp(P->cached.data(), grads_host, sizeof(void*) * P->n_tensors) == 0)
+        return 0;
+    // A captured write runs at each replay, whatever was uploaded before or in
+    // between: it is always recorded, with the pointers in the graph itself
+    // (a pinned buffer would have to stay unchanged as long as the graph),
+    // and from then on the plan's own record says nothing about the table.
+    if (capturing || P->n_tensors <= kArgGrads) {
+        P->table_captured |= capturing;
+        for (int32_t at = 0; at < P->n_tensors; at += kArgGrads) {
+            const int32_t n = std::min(P->n_tensors - at, kArgGrads);
+            GradTable t{};
+            std::memcpy(t.p, grads_host + at, sizeof(void*) * n);
+            hipLaunchKernelGGL(write_grads_kernel, dim3(1), dim3(kBlock), 0, s, t, n, P->d_grads + at);
+            if (int rc = launch_check("write_grads_kernel")) return rc;
+        }
     } else {
         const int k = P->slot;
         // The staging slot may still feed an earlier copy; its event says when it is free.
