@@ -26,6 +26,10 @@ from .adamw import _OWNER, engine_of
 #: plans of gradient sets no engine owns, by the set's key: the device index, then each gradient's length (8 bytes)
 #: and dtype code (1 byte)
 _GRAD_PLANS: dict[bytes, int] = {}
+#: the plans that captured calls use, by the same key: a graph holds the addresses of a plan's device tables, so a plan
+#: once captured is never given back, and calls outside a capture leave it to the replays (its gradient table is then
+#: the graph's).  One per set, shared by all captures of it.
+_CAPTURED_PLANS: dict[bytes, int] = {}
 _last_fast: tuple[tuple, weakref.ref] | None = None   # (id tuple, engine) of the last fused-path call
 
 
@@ -66,12 +70,32 @@ def _grad_plan(key: bytes) -> int:
     return plan.value
 
 
+def _capturing(index: int) -> bool:
+    """Whether torch's current stream on GPU `index` is capturing a graph."""
+    if index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(index):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def _plan_for(key: bytes, index: int) -> int:
+    if not _capturing(index):
+        plan = _GRAD_PLANS.get(key)
+        return _grad_plan(key) if plan is None else plan
+    plan = _CAPTURED_PLANS.get(key)
+    if plan is None:
+        plan = _GRAD_PLANS.pop(key, None)
+        if plan is None:
+            raise RuntimeError("run clip_grad_norm_ once on gradients of these lengths and dtypes outside graph "
+                               "capture before capturing it")
+        _CAPTURED_PLANS[key] = plan
+    return plan
+
+
 def _norm_only(table: tuple[bytes, bytes, int], max_norm: float, error_if_nonfinite: bool) -> torch.Tensor:
     key, ptrs, index = table
     N.lib()
-    plan = _GRAD_PLANS.get(key)
-    if plan is None:
-        plan = _grad_plan(key)
+    plan = _plan_for(key, index)
     stream = N.stream_handle(index)
     # torch checks finiteness (clip_grad.py:110-116) before it scales (:232)
     scale = 0 if error_if_nonfinite else N.entry_address("mgopt_scale_grads")
@@ -96,7 +120,12 @@ def clip_grad_norm_(
     """Total L2 norm of the gradients (as one vector), clipping them to
     max_norm: coefficient min(1, max_norm / (norm + 1e-6)), applied with no
     host branch (clip_grad.py:185-233).  Returns the pre-clip norm as a 0-dim
-    float32 tensor on the GPU."""
+    float32 tensor on the GPU.
+
+    In a graph capture, a list that is not an optimizer's needs one call
+    before it, on gradients of the same lengths and dtypes.  Graphs that clip
+    such sets share one plan: their replays must not overlap, nor the first
+    of them a call that began before the capture."""
     if float(norm_type) != 2.0:
         raise NotImplementedError("only norm_type=2.0 is implemented")
     if isinstance(parameters, torch.Tensor):

@@ -1,0 +1,119 @@
+"""Which plan a stand-alone clip_grad_norm_ takes, and what it launches on it:
+the native calls are replaced by a recorder, so nothing here needs a GPU."""
+
+from __future__ import annotations
+
+import contextlib
+import ctypes
+import importlib
+import struct
+
+import pytest
+import torch
+
+clip = importlib.import_module("minigpt-train-infra_amd.clip_grad")
+N = clip.N
+
+
+class _Native:
+    """Stands for the library and the host helper."""
+
+    def __init__(self):
+        self.capturing, self.stream = False, 0
+        self.created = 0
+        self.alive: set[int] = set()
+        self.calls: list[tuple] = []        # (what, plan, first gradient pointer or None, stream)
+
+    # the library
+    def mgopt_plan_create(self, descs, n, groups, steps, chunk, out):
+        if self.capturing:
+            return 900                      # hipErrorStreamCaptureUnsupported: a plan allocates
+        self.created += 1
+        out._obj.value = 0x1000 * self.created
+        self.alive.add(out._obj.value)
+        return 0
+
+    def mgopt_plan_destroy(self, plan):
+        self.alive.remove(getattr(plan, "value", plan))
+        return 0
+
+    def mgopt_plan_set_grads(self, plan, table, stream):
+        self.calls.append(("set", plan, ctypes.cast(table, ctypes.POINTER(ctypes.c_uint64))[0], stream))
+        return 0
+
+    def mgopt_scale_grads(self, plan, coef, stream):
+        self.calls.append(("scale", plan, None, stream))
+        return 0
+
+    def mgopt_last_error(self):
+        return b"refused"
+
+    # the host helper
+    def clip_launch(self, set_fn, norm_fn, scale_fn, plan, ptrs, max_norm, index, stream):
+        assert plan in self.alive
+        self.calls.append(("set", plan, struct.unpack_from("<Q", ptrs)[0], stream))
+        if scale_fn:
+            self.calls.append(("scale", plan, None, stream))
+        return 0, torch.zeros(()), torch.zeros(())
+
+    @property
+    def plans(self):
+        return [c[1] for c in self.calls if c[0] == "set"]
+
+
+@pytest.fixture
+def native(monkeypatch):
+    f = _Native()
+    monkeypatch.setattr(N, "lib", lambda: f)
+    monkeypatch.setattr(N, "load_library", lambda: f)
+    monkeypatch.setattr(N, "host", lambda: f)
+    monkeypatch.setattr(N, "entry_address", lambda name: 1)
+    monkeypatch.setattr(N, "stream_handle", lambda device: f.stream)
+    monkeypatch.setattr(torch.cuda, "device", lambda index: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: f.capturing)
+    for name in ("_GRAD_PLANS", "_CAPTURED_PLANS"):
+        monkeypatch.setattr(clip, name, {}, raising=False)
+    return f
+
+
+def _table(numel, first=0x100, device=0):
+    """What the host helper's clip_table returns for one fp32 gradient."""
+    return struct.pack("<qqb", device, numel, 0), struct.pack("<Q", first), device
+
+
+def _clip(native, numel, first=0x100, **kw):
+    """One call; returns the plan it ran on."""
+    clip._norm_only(_table(numel, first), 1.0, kw.get("error_if_nonfinite", False))
+    return native.plans[-1]
+
+
+def test_remembered_sets_are_bounded(native):
+    plans = [_clip(native, 10 + k) for k in range(40)]
+    assert len(set(plans)) == 40 and len(native.alive) == 17
+    assert _clip(native, 49) == plans[39]
+
+
+def test_a_captured_plan_is_the_graphs(native):
+    """Calls outside the graph take another plan, further captures the same
+    one, and no number of other sets gives it back."""
+    warm = _clip(native, 10)
+    native.capturing = True
+    captured = _clip(native, 10)
+    assert captured == warm
+    native.capturing = False
+    eager = _clip(native, 10)
+    assert eager != captured and _clip(native, 10) == eager
+    native.capturing = True
+    assert _clip(native, 10) == captured
+    native.capturing = False
+    for k in range(40):
+        _clip(native, 100 + k)
+    assert captured in native.alive and eager not in native.alive
+
+
+def test_capture_without_a_plan_is_refused(native):
+    native.capturing = True
+    with pytest.raises(RuntimeError, match="outside graph capture"):
+        _clip(native, 10)
+    assert native.calls == []

@@ -1,0 +1,98 @@
+"""The plans of a stand-alone clip_grad_norm_ on the GPU: graph replays between
+calls outside the graph.  Expected values are the oracle's norm and each
+gradient times the coefficient in fp32, rounded once to its dtype."""
+
+from __future__ import annotations
+
+import importlib
+
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests._gpu_harness import log
+
+pytestmark = pytest.mark.gpu
+
+mg = importlib.import_module("minigpt-train-infra_amd")
+DEV = "cuda:0"
+
+
+class _Set:
+    """Parameters with gradients, and what one clip to `max_norm` makes of them."""
+
+    def __init__(self, sizes, dtype, seed, sigma, max_norm=0.25):
+        gen = torch.Generator(device=DEV).manual_seed(seed)
+        self.max_norm = max_norm
+        self.first = [torch.empty(n, device=DEV).normal_(0.0, sigma, generator=gen).to(dtype) for n in sizes]
+        self.params = [torch.nn.Parameter(torch.empty_like(g)) for g in self.first]
+        for p, g in zip(self.params, self.first):
+            p.grad = g.clone()
+        self.norm = O.norm_from_sumsq(sum(O.sumsq(g.float().cpu().numpy()) for g in self.first))
+        coef = torch.tensor(O.clip_coef(self.norm, max_norm), dtype=torch.float32, device=DEV)
+        self.want = [(g.float() * coef).to(g.dtype) for g in self.first]
+
+    def reset(self):
+        for p, g in zip(self.params, self.first):
+            p.grad.copy_(g)
+
+    def clip(self):
+        return mg.clip_grad_norm_(self.params, self.max_norm)
+
+    def check(self, norm, clipped=True):
+        assert float(norm) == self.norm
+        for p, g in zip(self.params, self.want if clipped else self.first):
+            assert torch.equal(p.grad, g)
+
+
+@pytest.mark.parametrize("count", [3, 480, 481])
+def test_replays_and_calls_outside_the_graph(count):
+    """One set captured, another of the same lengths clipped in between, and
+    20 sets of other lengths, more than are remembered."""
+    log(f"case: captured clip of {count} gradients")
+    sizes = [1 + k % 700 for k in range(count)]
+    mine, other = (_Set(sizes, torch.float32, seed, sigma) for seed, sigma in ((1, 1.0), (2, 3.0)))
+    other.check(other.clip())           # the warm-up, on other gradients than the captured ones
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = mine.clip()
+    for k in range(3):
+        other.reset()
+        other.check(other.clip())
+        mine.reset()
+        graph.replay()
+        mine.check(captured)
+        mine.reset()
+        mine.check(mine.clip())         # the captured gradients, outside the graph
+        if k == 0:
+            for n in range(20):
+                extra = _Set([2000 + n], torch.float32, n, 1.0)
+                extra.check(extra.clip())
+
+
+@pytest.mark.parametrize("count", [479, 480, 481])
+def test_buffers_replaced_between_calls(count):
+    """Around the length at which the gradient table's upload changes form."""
+    log(f"case: clip of {count} gradients in new buffers")
+    sizes = [1 + k % 100 for k in range(count)]
+    sets = [_Set(sizes, torch.bfloat16, seed, 1.0 + seed) for seed in range(6)]
+    norms = [s.clip() for s in sets]
+    for s, norm in zip(sets, norms):
+        s.check(norm)
+
+
+def test_capture_before_any_call_is_refused():
+    fresh = _Set([4321], torch.float32, 5, 1.0)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        graph.capture_begin()
+        try:
+            with pytest.raises(RuntimeError, match="outside graph capture"):
+                fresh.clip()
+        finally:
+            graph.capture_end()
+    torch.cuda.synchronize()
+    assert torch.equal(fresh.params[0].grad, fresh.first[0])
+    fresh.check(fresh.clip())
