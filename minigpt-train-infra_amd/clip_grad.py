@@ -23,10 +23,14 @@ import torch
 from . import _native as N
 from .adamw import _OWNER, engine_of
 
-#: plans of gradient sets no engine owns, by the set's key: the device index, then each gradient's length (8 bytes)
-#: and dtype code (1 byte)
-_GRAD_PLANS: dict[bytes, int] = {}
-#: the plans that captured calls use, by the same key: a graph holds the addresses of a plan's device tables, so a plan
+#: plans of gradient sets no engine owns, by the set's key (the device index, then each gradient's length in 8 bytes
+#: and dtype code in 1) and by stream: a plan holds the gradient table, the partials and the ticket counter of the call
+#: in flight, so calls on two streams need one each.  A plan's tables take about 0.3 % of the gradients' bytes and
+#: 120-250 bytes per tensor, outside torch's allocator.
+_GRAD_PLANS: dict[bytes, dict[int, int]] = {}
+MAX_SETS = 17
+MAX_STREAMS = 33       # per set: torch's pool of 32 and the default stream
+#: the plans that captured calls use, by the set's key: a graph holds the addresses of a plan's device tables, so a plan
 #: once captured is never given back, and calls outside a capture leave it to the replays (its gradient table is then
 #: the graph's).  One per set, shared by all captures of it.
 _CAPTURED_PLANS: dict[bytes, int] = {}
@@ -48,8 +52,10 @@ def _grad_table(grads: list[torch.Tensor]) -> tuple[bytes, bytes, int]:
     return key, struct.pack(f"<{len(grads)}Q", *(g.data_ptr() for g in grads)), dev.index
 
 
-def _grad_plan(key: bytes) -> int:
-    """A new plan for the gradient set of `key`; the oldest of more than 17 is given back."""
+def _grad_plan(key: bytes, stream: int) -> int:
+    """A new plan for calls on `stream` with the gradient set of `key`; the
+    oldest set's plans, and the set's oldest one, are given back above the
+    limits."""
     lib = N.lib()
     index, = struct.unpack_from("<q", key)
     sets = list(struct.iter_unpack("<qb", key[8:]))
@@ -64,9 +70,13 @@ def _grad_plan(key: bytes) -> int:
     plan = ctypes.c_void_p()
     with torch.cuda.device(index):
         N.check(lib.mgopt_plan_create(descs, len(sets), 1, None, chunk, ctypes.byref(plan)), "mgopt_plan_create")
-    if len(_GRAD_PLANS) > 16:
-        lib.mgopt_plan_destroy(ctypes.c_void_p(_GRAD_PLANS.pop(next(iter(_GRAD_PLANS)))))
-    _GRAD_PLANS[key] = plan.value
+    by_stream = _GRAD_PLANS.setdefault(key, {})
+    by_stream[stream] = plan.value
+    old = [by_stream.pop(next(iter(by_stream)))] if len(by_stream) > MAX_STREAMS else []
+    if len(_GRAD_PLANS) > MAX_SETS:
+        old += _GRAD_PLANS.pop(next(iter(_GRAD_PLANS))).values()
+    for handle in old:
+        lib.mgopt_plan_destroy(ctypes.c_void_p(handle))
     return plan.value
 
 
@@ -78,25 +88,26 @@ def _capturing(index: int) -> bool:
         return torch.cuda.is_current_stream_capturing()
 
 
-def _plan_for(key: bytes, index: int) -> int:
+def _plan_for(key: bytes, index: int, stream: int) -> int:
     if not _capturing(index):
-        plan = _GRAD_PLANS.get(key)
-        return _grad_plan(key) if plan is None else plan
+        plan = _GRAD_PLANS.get(key, {}).get(stream)
+        return _grad_plan(key, stream) if plan is None else plan
     plan = _CAPTURED_PLANS.get(key)
     if plan is None:
-        plan = _GRAD_PLANS.pop(key, None)
-        if plan is None:
+        by_stream = _GRAD_PLANS.get(key)
+        if not by_stream:
             raise RuntimeError("run clip_grad_norm_ once on gradients of these lengths and dtypes outside graph "
                                "capture before capturing it")
-        _CAPTURED_PLANS[key] = plan
+        # a capture has a stream of its own as a rule: the set's newest plan then
+        plan = _CAPTURED_PLANS[key] = by_stream.pop(stream if stream in by_stream else next(reversed(by_stream)))
     return plan
 
 
 def _norm_only(table: tuple[bytes, bytes, int], max_norm: float, error_if_nonfinite: bool) -> torch.Tensor:
     key, ptrs, index = table
     N.lib()
-    plan = _plan_for(key, index)
     stream = N.stream_handle(index)
+    plan = _plan_for(key, index, stream)
     # torch checks finiteness (clip_grad.py:110-116) before it scales (:232)
     scale = 0 if error_if_nonfinite else N.entry_address("mgopt_scale_grads")
     rc, norm, coef = N.host().clip_launch(N.entry_address("mgopt_plan_set_grads"), N.entry_address("mgopt_grad_norm"),

@@ -112,6 +112,31 @@ def test_a_captured_plan_is_the_graphs(native):
     assert captured in native.alive and eager not in native.alive
 
 
+def test_each_stream_has_its_own_plan(native):
+    """The plan holds the table, the partials and the tickets of one call, so
+    calls that may overlap share none of them."""
+    plans = []
+    for native.stream in (0, 7, 8):
+        plans.append(_clip(native, 10))
+    assert len(set(plans)) == 3
+    for native.stream, plan in zip((0, 7, 8), plans):
+        assert _clip(native, 10) == plan
+    native.stream, native.capturing = 9, True       # a capture's own stream: the newest
+    assert _clip(native, 10) == plans[2]
+    native.stream, native.capturing = 7, False
+    assert _clip(native, 10) == plans[1]
+
+
+def test_plans_per_stream_are_bounded(native):
+    for native.stream in range(100):
+        _clip(native, 10)
+    assert len(native.alive) == 33
+    native.stream = 0
+    for k in range(17):
+        _clip(native, 100 + k)
+    assert len(native.alive) == 17
+
+
 def test_capture_without_a_plan_is_refused(native):
     native.capturing = True
     with pytest.raises(RuntimeError, match="outside graph capture"):

@@ -1,5 +1,5 @@
 """The plans of a stand-alone clip_grad_norm_ on the GPU: graph replays between
-calls outside the graph.  Expected values are the oracle's norm and each
+calls outside the graph, and calls on several streams.  Expected values are the oracle's norm and each
 gradient times the coefficient in fp32, rounded once to its dtype."""
 
 from __future__ import annotations
@@ -96,3 +96,24 @@ def test_capture_before_any_call_is_refused():
     torch.cuda.synchronize()
     assert torch.equal(fresh.params[0].grad, fresh.first[0])
     fresh.check(fresh.clip())
+
+
+@pytest.mark.parametrize("sizes,dtype", [
+    ([700_000, 5, 300_001], torch.float32),             # the finalize in pass 1's last work-group
+    ([4_000_003] * 3, torch.bfloat16),
+    ([1 + k % 900 for k in range(1000)], torch.float32),   # the gradient table copied from a pinned buffer
+], ids=["folded", "five-kernels", "long-table"])
+def test_same_lengths_on_two_streams(sizes, dtype):
+    log(f"case: two streams, {len(sizes)} gradients")
+    sets = [_Set(sizes, dtype, seed, 1.0 + seed) for seed in range(4)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for rep in range(5):
+        norms = []
+        for k, s in enumerate(sets):                    # sets 0 and 2 on one stream, 1 and 3 on the other
+            with torch.cuda.stream(streams[k % 2]):
+                s.reset()
+                norms.append(s.clip())
+        torch.cuda.synchronize()
+        for s, norm in zip(sets, norms):
+            s.check(norm)
