@@ -13,6 +13,8 @@ from __future__ import annotations
 
 import ctypes
 import struct
+import sys
+import threading
 import types
 import warnings
 import weakref
@@ -23,17 +25,50 @@ import torch
 from . import _native as N
 from .adamw import _OWNER, engine_of
 
+class _GradPlan:
+    """A plan of gradients no engine owns, for the set of `key`.  Whoever holds
+    it keeps it alive, so a call may use the plan it looked up whatever other
+    threads remember meanwhile; its lock is held from a gradient table to the
+    last launch that reads it."""
+
+    __slots__ = ("handle", "lock")
+
+    def __init__(self, key: bytes):
+        self.handle, self.lock = None, threading.Lock()
+        index, = struct.unpack_from("<q", key)
+        sets = list(struct.iter_unpack("<qb", key[8:]))
+        descs = (N.TensorDesc * len(sets))()
+        for d, (numel, code) in zip(descs, sets):
+            d.numel = numel
+            d.group = 0
+            d.grad_dtype = code
+            d.lowp_dtype = N.NONE
+        # elements per work-group of the in-place scaling: 4 KB of gradients (mgopt.hip, scale_grads_kernel)
+        chunk = 1024 if any(code == N.F32 for _, code in sets) else 2048
+        plan = ctypes.c_void_p()
+        with torch.cuda.device(index):
+            N.check(N.lib().mgopt_plan_create(descs, len(sets), 1, None, chunk, ctypes.byref(plan)),
+                    "mgopt_plan_create")
+        self.handle = plan.value
+
+    def __del__(self, _finalizing=sys.is_finalizing):
+        # bound at class definition: at interpreter shutdown the process releases everything itself
+        if self.handle is not None and not _finalizing():
+            N.load_library().mgopt_plan_destroy(ctypes.c_void_p(self.handle))
+
+
 #: plans of gradient sets no engine owns, by the set's key (the device index, then each gradient's length in 8 bytes
 #: and dtype code in 1) and by stream: a plan holds the gradient table, the partials and the ticket counter of the call
 #: in flight, so calls on two streams need one each.  A plan's tables take about 0.3 % of the gradients' bytes and
 #: 120-250 bytes per tensor, outside torch's allocator.
-_GRAD_PLANS: dict[bytes, dict[int, int]] = {}
+_GRAD_PLANS: dict[bytes, dict[int, _GradPlan]] = {}
 MAX_SETS = 17
 MAX_STREAMS = 33       # per set: torch's pool of 32 and the default stream
 #: the plans that captured calls use, by the set's key: a graph holds the addresses of a plan's device tables, so a plan
 #: once captured is never given back, and calls outside a capture leave it to the replays (its gradient table is then
 #: the graph's).  One per set, shared by all captures of it.
-_CAPTURED_PLANS: dict[bytes, int] = {}
+_CAPTURED_PLANS: dict[bytes, _GradPlan] = {}
+_PLANS_LOCK = threading.Lock()   # changes of these two
 _last_fast: tuple[tuple, weakref.ref] | None = None   # (id tuple, engine) of the last fused-path call
 
 
@@ -52,34 +87,6 @@ def _grad_table(grads: list[torch.Tensor]) -> tuple[bytes, bytes, int]:
     return key, struct.pack(f"<{len(grads)}Q", *(g.data_ptr() for g in grads)), dev.index
 
 
-def _grad_plan(key: bytes, stream: int) -> int:
-    """A new plan for calls on `stream` with the gradient set of `key`; the
-    oldest set's plans, and the set's oldest one, are given back above the
-    limits."""
-    lib = N.lib()
-    index, = struct.unpack_from("<q", key)
-    sets = list(struct.iter_unpack("<qb", key[8:]))
-    descs = (N.TensorDesc * len(sets))()
-    for d, (numel, code) in zip(descs, sets):
-        d.numel = numel
-        d.group = 0
-        d.grad_dtype = code
-        d.lowp_dtype = N.NONE
-    # elements per work-group of the in-place scaling: 4 KB of gradients (mgopt.hip, scale_grads_kernel)
-    chunk = 1024 if any(code == N.F32 for _, code in sets) else 2048
-    plan = ctypes.c_void_p()
-    with torch.cuda.device(index):
-        N.check(lib.mgopt_plan_create(descs, len(sets), 1, None, chunk, ctypes.byref(plan)), "mgopt_plan_create")
-    by_stream = _GRAD_PLANS.setdefault(key, {})
-    by_stream[stream] = plan.value
-    old = [by_stream.pop(next(iter(by_stream)))] if len(by_stream) > MAX_STREAMS else []
-    if len(_GRAD_PLANS) > MAX_SETS:
-        old += _GRAD_PLANS.pop(next(iter(_GRAD_PLANS))).values()
-    for handle in old:
-        lib.mgopt_plan_destroy(ctypes.c_void_p(handle))
-    return plan.value
-
-
 def _capturing(index: int) -> bool:
     """Whether torch's current stream on GPU `index` is capturing a graph."""
     if index == torch.cuda.current_device():
@@ -88,18 +95,40 @@ def _capturing(index: int) -> bool:
         return torch.cuda.is_current_stream_capturing()
 
 
-def _plan_for(key: bytes, index: int, stream: int) -> int:
-    if not _capturing(index):
-        plan = _GRAD_PLANS.get(key, {}).get(stream)
-        return _grad_plan(key, stream) if plan is None else plan
-    plan = _CAPTURED_PLANS.get(key)
-    if plan is None:
-        by_stream = _GRAD_PLANS.get(key)
-        if not by_stream:
-            raise RuntimeError("run clip_grad_norm_ once on gradients of these lengths and dtypes outside graph "
-                               "capture before capturing it")
-        # a capture has a stream of its own as a rule: the set's newest plan then
-        plan = _CAPTURED_PLANS[key] = by_stream.pop(stream if stream in by_stream else next(reversed(by_stream)))
+def _plan_for(key: bytes, index: int, stream: int) -> _GradPlan:
+    if _capturing(index):
+        return _captured_plan(key, stream)
+    by_stream = _GRAD_PLANS.get(key)
+    plan = by_stream.get(stream) if by_stream is not None else None
+    return _new_plan(key, stream) if plan is None else plan
+
+
+def _new_plan(key: bytes, stream: int) -> _GradPlan:
+    """A new plan, remembered for calls on `stream`; the set's oldest plan, and
+    the oldest set's plans, are given back above the limits."""
+    plan, old = _GradPlan(key), []
+    with _PLANS_LOCK:
+        by_stream = _GRAD_PLANS.setdefault(key, {})
+        old.append(by_stream.pop(stream, None))      # another thread's, made meanwhile
+        by_stream[stream] = plan
+        if len(by_stream) > MAX_STREAMS:
+            old.append(by_stream.pop(next(iter(by_stream))))
+        if len(_GRAD_PLANS) > MAX_SETS:
+            old.append(_GRAD_PLANS.pop(next(iter(_GRAD_PLANS))))
+    return plan                                      # `old` goes here, outside the lock: that waits for the GPU
+
+
+def _captured_plan(key: bytes, stream: int) -> _GradPlan:
+    with _PLANS_LOCK:
+        plan = _CAPTURED_PLANS.get(key)
+        if plan is None:
+            by_stream = _GRAD_PLANS.get(key)
+            if not by_stream:
+                raise RuntimeError("run clip_grad_norm_ once on gradients of these lengths and dtypes outside graph "
+                                   "capture before capturing it")
+            # a capture has a stream of its own as a rule: the set's newest plan then
+            plan = by_stream.pop(stream if stream in by_stream else next(reversed(by_stream)))
+            _CAPTURED_PLANS[key] = plan
     return plan
 
 
@@ -110,12 +139,18 @@ def _norm_only(table: tuple[bytes, bytes, int], max_norm: float, error_if_nonfin
     plan = _plan_for(key, index, stream)
     # torch checks finiteness (clip_grad.py:110-116) before it scales (:232)
     scale = 0 if error_if_nonfinite else N.entry_address("mgopt_scale_grads")
-    rc, norm, coef = N.host().clip_launch(N.entry_address("mgopt_plan_set_grads"), N.entry_address("mgopt_grad_norm"),
-                                          scale, plan, ptrs, max_norm, index, stream)
-    N.check(rc, "clip_grad_norm_")
+    with plan.lock:
+        rc, norm, coef = N.host().clip_launch(N.entry_address("mgopt_plan_set_grads"),
+                                              N.entry_address("mgopt_grad_norm"), scale, plan.handle, ptrs, max_norm,
+                                              index, stream)
+        N.check(rc, "clip_grad_norm_")
     if error_if_nonfinite:
         _check_finite(norm, error_if_nonfinite)
-        N.check(N.lib().mgopt_scale_grads(plan, coef.data_ptr(), stream), "mgopt_scale_grads")
+        grads = ctypes.cast(ctypes.c_char_p(ptrs), ctypes.POINTER(ctypes.c_void_p))
+        with plan.lock:
+            # once more: another thread's call may have used the plan while this one waited
+            N.check(N.lib().mgopt_plan_set_grads(plan.handle, grads, stream), "mgopt_plan_set_grads")
+            N.check(N.lib().mgopt_scale_grads(plan.handle, coef.data_ptr(), stream), "mgopt_scale_grads")
     return norm
 
 

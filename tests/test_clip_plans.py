@@ -42,7 +42,7 @@ class _Native:
         return 0
 
     def mgopt_scale_grads(self, plan, coef, stream):
-        self.calls.append(("scale", plan, None, stream))
+        self.calls.append(("scale" if plan in self.alive else "scale-after-free", plan, None, stream))
         return 0
 
     def mgopt_last_error(self):
@@ -135,6 +135,30 @@ def test_plans_per_stream_are_bounded(native):
     for k in range(17):
         _clip(native, 100 + k)
     assert len(native.alive) == 17
+
+
+def test_another_call_during_the_finiteness_check(native, monkeypatch):
+    """error_if_nonfinite=True waits for the norm before it scales.  Calls
+    made meanwhile, on the same lengths (another gradient table) and on other
+    lengths (which push the plan out of memory), must not change what it
+    scales."""
+    check, nested = clip._check_finite, []
+
+    def check_after_others(total, error_if_nonfinite, eng=None):
+        if error_if_nonfinite and not nested:
+            nested.append(True)
+            _clip(native, 10, first=0x900)
+            for k in range(40):
+                _clip(native, 100 + k)
+        check(total, error_if_nonfinite, eng)
+
+    monkeypatch.setattr(clip, "_check_finite", check_after_others)
+    clip._norm_only(_table(10, 0x500), 1.0, True)
+    assert nested
+    what, plan, _, _ = native.calls[-1]
+    assert what == "scale" and plan == native.plans[0]
+    assert [c[2] for c in native.calls if c[:2] == ("set", plan)][-1] == 0x500
+    assert all(c[0] != "scale-after-free" for c in native.calls)
 
 
 def test_capture_without_a_plan_is_refused(native):

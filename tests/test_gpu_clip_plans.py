@@ -1,10 +1,12 @@
 """The plans of a stand-alone clip_grad_norm_ on the GPU: graph replays between
-calls outside the graph, and calls on several streams.  Expected values are the oracle's norm and each
-gradient times the coefficient in fp32, rounded once to its dtype."""
+calls outside the graph, calls on several streams and from several threads.
+Expected values are the oracle's norm and each gradient times the coefficient
+in fp32, rounded once to its dtype."""
 
 from __future__ import annotations
 
 import importlib
+import threading
 
 import pytest
 import torch
@@ -117,3 +119,27 @@ def test_same_lengths_on_two_streams(sizes, dtype):
         torch.cuda.synchronize()
         for s, norm in zip(sets, norms):
             s.check(norm)
+
+
+def test_threads_share_lengths_and_a_stream():
+    """Four threads clip sets of the same lengths on the default stream at
+    once, half of them with error_if_nonfinite=True (which waits for the GPU
+    between the norm and the scaling)."""
+    log("case: four threads on one stream")
+    sets = [_Set([1 + k % 300 for k in range(600)], torch.float32, seed, 1.0 + seed) for seed in range(4)]
+    norms = [[] for _ in sets]
+
+    def work(k):
+        for _ in range(10):
+            sets[k].reset()
+            norms[k].append(mg.clip_grad_norm_(sets[k].params, 0.25, error_if_nonfinite=k % 2 == 0))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(sets))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for s, got in zip(sets, norms):
+        assert [float(x) for x in got] == [s.norm] * 10
+        s.check(got[-1])
