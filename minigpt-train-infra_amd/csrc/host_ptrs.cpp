@@ -239,17 +239,23 @@ py::object clip_table(const py::list& params) {
 }
 
 // clip_grad_norm_'s launches on such a set: the gradient table, the norm and,
-// with scale_fn, the scaling.  Returns (status, norm, coefficient).
+// with scale_fn, the scaling.  Returns (status, norm, coefficient).  The upload
+// of a long table may wait for the GPU, so other Python threads run meanwhile.
 py::tuple clip_launch(uint64_t set_fn, uint64_t norm_fn, uint64_t scale_fn, uint64_t plan, const std::string& ptrs,
                       double max_norm, int64_t device, uint64_t stream) {
     const auto options = at::TensorOptions().dtype(at::kFloat).device(c10::kCUDA, static_cast<c10::DeviceIndex>(device));
     const at::Tensor norm = at::empty({}, options), coef = at::empty({}, options);
+    float* const n = norm.data_ptr<float>();
+    float* const c = coef.data_ptr<float>();
     void* const p = as_ptr<void*>(plan);
     void* const s = as_ptr<void*>(stream);
-    int rc = as_ptr<SetGradsFn>(set_fn)(p, reinterpret_cast<const void* const*>(ptrs.data()), s);
-    if (rc == 0)
-        rc = as_ptr<GradNormFn>(norm_fn)(p, nullptr, max_norm, norm.data_ptr<float>(), coef.data_ptr<float>(), nullptr, s);
-    if (rc == 0 && scale_fn != 0) rc = as_ptr<ScaleGradsFn>(scale_fn)(p, coef.data_ptr<float>(), s);
+    int rc;
+    {
+        py::gil_scoped_release others;
+        rc = as_ptr<SetGradsFn>(set_fn)(p, reinterpret_cast<const void* const*>(ptrs.data()), s);
+        if (rc == 0) rc = as_ptr<GradNormFn>(norm_fn)(p, nullptr, max_norm, n, c, nullptr, s);
+        if (rc == 0 && scale_fn != 0) rc = as_ptr<ScaleGradsFn>(scale_fn)(p, c, s);
+    }
     return py::make_tuple(rc, norm, coef);
 }
 
