@@ -182,8 +182,8 @@ MGOPT_API int mgopt_adamw_step(mgopt_plan* plan, const mgopt_group_hparams* grou
 /* Writes n_groups hyper-parameter sets to dst_dev (8-byte aligned, on GPU
  * `device`), the array that a step with MGOPT_GROUPS_ON_DEVICE reads, in stream
  * order: replays enqueued before it on `stream` still read the earlier
- * records.  `groups` is read before the call returns.  No reference
- * counterpart. */
+ * records.  `groups` is read before the call returns.  MGOPT_E_INVALID where
+ * there is no GPU `device`.  No reference counterpart. */
 MGOPT_API int mgopt_write_groups(int32_t device, const mgopt_group_hparams* groups, int32_t n_groups, void* dst_dev,
                                  void* stream);
 

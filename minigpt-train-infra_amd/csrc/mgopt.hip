@@ -1291,10 +1291,13 @@ int hip_fail(hipError_t e, const char* what) {
 struct DeviceGuard {
     int prev = -1;
     bool switched = false;
+    bool current = false;  // `dev` is the current device: false where there is no such device
     explicit DeviceGuard(int dev) {
         // restores the caller's device only when it had to switch: the common
         // case (the plan's device is current) costs one hipGetDevice
         if (hipGetDevice(&prev) == hipSuccess && prev != dev) switched = hipSetDevice(dev) == hipSuccess;
+        current = prev == dev || switched;
+        if (!current) (void)hipGetLastError();  // or a later launch would report it
     }
     ~DeviceGuard() {
         if (switched) (void)hipSetDevice(prev);
@@ -1857,6 +1860,7 @@ MGOPT_API int mgopt_write_groups(int32_t device, const mgopt_group_hparams* grou
     if (n_groups <= 0 || n_groups > MGOPT_MAX_GROUPS) return fail(MGOPT_E_LIMIT, "n_groups must be in 1..16");
     if (reinterpret_cast<uintptr_t>(dst_dev) % 8 != 0) return fail(MGOPT_E_ALIGN, "records must be 8-byte aligned");
     DeviceGuard guard(device);
+    if (device < 0 || !guard.current) return fail(MGOPT_E_INVALID, "no device " + std::to_string(device));
     GroupRecords r{};
     std::memcpy(r.g, groups, sizeof(GroupConst) * n_groups);
     hipLaunchKernelGGL(write_groups_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), r,

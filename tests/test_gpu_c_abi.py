@@ -292,3 +292,19 @@ def test_hyperparameters_from_device_memory_match_by_value():
     finally:
         lib.mgopt_plan_destroy(a[0])
         lib.mgopt_plan_destroy(b[0])
+
+
+def test_group_records_for_a_device_that_is_not_there():
+    """Refused before a launch: the records stay, nothing is left in HIP's
+    last error, and the next call writes them."""
+    lib = _lib()
+    lib.mgopt_write_groups.argtypes = [ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p]
+    log("case: group records, bad device index")
+    hp = (GroupHparams * 2)()
+    hp[0].lr, hp[1].eps = 3e-4, 1e-8
+    dst = torch.full((12,), -1.0, dtype=torch.float64, device=DEV)
+    for device in (-1, torch.cuda.device_count()):
+        assert lib.mgopt_write_groups(device, hp, 2, dst.data_ptr(), _stream()) == 10001
+        assert bool((dst == -1.0).all()) and torch.cuda.current_device() == 0
+    _ok(lib.mgopt_write_groups(0, hp, 2, dst.data_ptr(), _stream()), lib, "write")
+    assert bytes(hp) == dst.cpu().numpy().tobytes()

@@ -183,6 +183,20 @@ def test_c_abi_rejects_bad_arguments_before_touching_the_gpu():
     assert lib.mgopt_plan_folded(None) == -1
 
 
+def test_write_groups_rejects_bad_arguments():
+    native = importlib.import_module("minigpt-train-infra_amd._native")
+    lib = native.load_library()
+    hp = (native.GroupHparams * 17)()
+    assert lib.mgopt_write_groups(0, None, 1, 0x1000, None) == 10001
+    assert lib.mgopt_write_groups(0, hp, 1, None, None) == 10001
+    for n in (0, -1, 17):
+        assert lib.mgopt_write_groups(0, hp, n, 0x1000, None) == 10003
+    assert lib.mgopt_write_groups(0, hp, 1, 0x1004, None) == 10002
+    for device in (-1, -(2 ** 31), 63, 2 ** 31 - 1):
+        assert lib.mgopt_write_groups(device, hp, 1, 0x1000, None) == 10001, device
+        assert f"no device {device}".encode() in lib.mgopt_last_error()
+
+
 def test_product_has_no_cpu_path(mg):
     p = nn.Parameter(torch.zeros(4))
     p.grad = torch.ones(4)
