@@ -1,5 +1,5 @@
 """clip_grad_norm_ over parameters no AdamW of the package owns: the in-place
-scaling in 4-KB chunks, with ordinary accesses up to 96 MiB of gradients and
+scaling in work-groups of 1 KB, with ordinary accesses up to 96 MiB of gradients and
 nontemporal ones above, 16-byte, 8-byte and single-element forms by alignment.
 Expected: each gradient times the returned norm's coefficient in fp32, rounded
 once to its dtype (what the kernel computes, so the comparison is exact)."""

@@ -11,9 +11,8 @@ copies and window record bit for bit: fp32, fp16 and bf16 gradients, fp16 and
 bf16 parameters with masters, tensors of one and of several chunks, an inf
 step, a parameter without a gradient for one step, a learning-rate schedule,
 a step count written in place beyond the bias-correction table, and written-
-back gradients.  The pass-1 chunkings differ (16,384 against 131,072
-elements), so the fp64 partial sums differ in rounding far below the fp32
-norm's; every norm is also checked against the oracle.
+back gradients.  Both forms sum the same pass-1 chunks of 16,384 elements
+in the same order; every norm is also checked against the oracle.
 """
 
 from __future__ import annotations

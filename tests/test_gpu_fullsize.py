@@ -217,14 +217,16 @@ def test_qwen3_8b_full_size():
 
 
 def test_pass2_beyond_one_dispatch():
-    """4.43e9 elements in 512-element chunks: 8,650,752 pass-2 work-groups,
-    more than one dispatch packet's 32-bit work-item count holds at 512
-    threads (8,388,607 work-groups), so pass 2 runs in two launches.  The
-    tensor holding the first chunk of the second launch, and the first and
+    """4.43e9 elements in 512-element chunks: 8,650,752 pass-2 chunks, more
+    than one launch takes (8,388,607 chunks by the cap every launch over the
+    chunk table has, 11,184,810 by the work-items of two 192-thread
+    work-groups per chunk), so pass 2 runs in two launches.  The tensor
+    holding the first chunk of the second launch, and the first and
     last tensors, are checked bit for bit against the oracle; every step count
     covers the rest.  fp32 params, fp16 grads, 62 GB."""
     shapes = [(f"w{i}", (4096, 4096)) for i in range(264)]
-    boundary = _tensor_at_chunk([s for _, s in shapes], 512, 0xFFFFFFFF // 512)
+    per_launch = min(0xFFFFFFFF // 512, 0xFFFFFFFF // 192 // (512 // 256))
+    boundary = _tensor_at_chunk([s for _, s in shapes], 512, per_launch)
     subset = sorted({0, boundary, len(shapes) - 1})
     log(f"case: 264 x 4096x4096 fp32/fp16, chunk 512, 2 steps, second launch starts in tensor {boundary}")
     pair = Pair(Case(shapes=shapes, param_dtype="f32", grad_dtype="f16", steps=2, sigma=1e-3, scaler=None,

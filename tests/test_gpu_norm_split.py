@@ -1,8 +1,10 @@
 """The split of pass 1 into chunks: norms of sets on both sides of each size
-at which the chunk length changes, with whole and ragged last chunks, against
-the oracle's compensated sum of squares.  The GPU's fp64 sums differ from it by
-under n * 2**-53 relative, far inside half an fp32 unit, so the rounded norms
-are equal."""
+at which the chunk length changes, with whole and ragged last chunks, and of
+flat buffers of the same lengths, against the oracle's compensated sum of
+squares.  The GPU adds at most 256 squares per thread of a chunk, 8 partials per
+thread of the finalize and 14 terms in the tree behind each, so its fp64 sums
+are off by under 320 * 2**-53 = 4e-14 relative, and the fp32 norms equal unless
+one lies that close to a rounding boundary."""
 
 from __future__ import annotations
 
@@ -13,6 +15,7 @@ import torch
 
 from oracle import oracle as O
 from tests._gpu_harness import log
+from tests.test_zz_no_alloc import _lib, _noalloc_norm
 
 pytestmark = pytest.mark.gpu
 
@@ -29,7 +32,7 @@ GROUPS, SHORTEST = 2048, 16384      # chunks a set is split into, shortest chunk
     (SHORTEST * GROUPS * 2 - 1,),                       # the next length, a ragged last chunk
     (3_000_000, 1, 8191, SHORTEST + 3, 2 * SHORTEST, 5),
 ], ids=lambda s: "+".join(map(str, s)))
-def test_norm_is_the_oracles_for_every_chunk_length(sizes, dtype):
+def test_norm_is_the_oracles_around_the_shorter_chunk_lengths(sizes, dtype):
     gen = torch.Generator(device=DEV).manual_seed(sum(sizes))
     params = []
     for n in sizes:
@@ -40,3 +43,22 @@ def test_norm_is_the_oracles_for_every_chunk_length(sizes, dtype):
     log(f"case: norm of {sizes} {dtype}")
     got = mg.clip_grad_norm_(params, 1e9)
     assert float(got) == want, (sizes, dtype, float(got), want)
+    if len(sizes) == 1:
+        assert _noalloc_norm(_lib(), params[0].grad, sizes[0], None, 1e9)[0] == want
+
+
+@pytest.mark.parametrize("length,dtype", [(65536, torch.float16), (131072, torch.bfloat16)])
+def test_the_longer_chunk_lengths(length, dtype):
+    """The two longest, each from 2,048 chunks of that length on: one chunk
+    fewer (the length before), and the first set with a ragged last one."""
+    full = length * GROUPS - 1
+    gen = torch.Generator(device=DEV).manual_seed(length)
+    p = torch.nn.Parameter(torch.empty(full, dtype=dtype, device=DEV))
+    g = torch.empty(full, dtype=dtype, device=DEV).normal_(0.0, 1e-2, generator=gen)
+    for n in (full - length + 1, full):
+        log(f"case: norm of {n} {dtype}")
+        q = torch.nn.Parameter(p.detach()[:n])
+        q.grad = g[:n]
+        want = O.norm_from_sumsq(O.sumsq(g[:n].float().cpu().numpy()))
+        assert float(mg.clip_grad_norm_([q], 1e9)) == want
+        assert _noalloc_norm(_lib(), g, n, None, 1e9)[0] == want

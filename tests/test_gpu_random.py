@@ -1,6 +1,6 @@
 """GPU parity on 24 seeded random configurations against the oracle: parameter
 dtype (fp32, or bf16 / fp16 with an fp32 master), gradient dtype, tensor sizes
-(1 element to several 131,072-element pass-1 chunks, odd sizes for the scalar
+(1 element to several 16,384-element pass-1 chunks, odd sizes for the scalar
 tails; the 4,096- and 65,536-element tensors as matrices whose state takes the
 row layout), chunk size, one or two groups with random betas (both lerp branches),
 eps, weight decay and maximize, a GradScaler with a random initial scale and

@@ -1,11 +1,11 @@
 """mgopt_grad_norm_noalloc through the C ABI: the allocation-free gradient norm
 of one flat gradient buffer against mgopt_grad_norm on a plan that holds the
-same buffer as its one tensor.  Both sum the same 131,072-element chunks into
-partials and finalize them in the same fixed order, so norm, clip
-coefficient and found_inf must agree bit for bit.  Two calls in a row, the
-second over a smaller buffer, show that the static partials array keeps no
-state a later call depends on; sizes above its maximum are refused.  Calls
-on either side of 256 MiB cover both of its load forms."""
+same buffer as its one tensor.  Both sum the same chunks into partials and
+finalize them in the same fixed order, so norm, clip coefficient and found_inf
+must agree bit for bit.  Two calls in a row, the second over a smaller buffer,
+show that the static partials array keeps no state a later call depends on;
+sizes above its maximum are refused.  Calls on either side of 256 MiB cover
+both of its load forms."""
 
 from __future__ import annotations
 
@@ -25,7 +25,7 @@ pytestmark = pytest.mark.gpu
 LIB_PATH = Path(__file__).resolve().parents[1] / "minigpt-train-infra_amd" / "_build" / "libmgopt.so"
 F32, F16, BF16, NONE = 0, 1, 2, -1
 E_INVALID, E_LIMIT = 10001, 10003
-MAX_ELEMS = 65536 * 131072          # 65,536 partials of 131,072-element chunks
+MAX_ELEMS = 65536 * 131072          # 65,536 partials of chunks of at most 131,072 elements
 DEV = "cuda:0"
 CODES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
@@ -63,8 +63,8 @@ def _stream():
 
 def _plan_norm(lib, g, scale, max_norm):
     """mgopt_grad_norm over a grads-only plan with `g` as its one tensor, in
-    the five-kernel form (MGOPT_FOLD=0), whose pass 1 sums the same
-    131,072-element chunks as the allocation-free norm."""
+    the five-kernel form (MGOPT_FOLD=0), whose pass 1 and finalize are those
+    of the allocation-free norm."""
     d = (TensorDesc * 1)()
     d[0].numel, d[0].group, d[0].grad_dtype, d[0].lowp_dtype = g.numel(), 0, CODES[g.dtype], NONE
     plan = ctypes.c_void_p()
@@ -132,8 +132,8 @@ def test_noalloc_norm_matches_the_plan_norm(dtype):
 def test_noalloc_norm_on_both_sides_of_the_cache_size():
     """Buffers of more than 256 MiB are read with nontemporal loads, smaller
     ones with loads that leave them in the Infinity Cache: one call just above
-    that size and one just below, each against the plan norm (whose plan picks
-    its loads by the same rule) and, for the sum of squares, against the
+    that size and one just below, each against the plan norm (whose plan, having
+    no optimizer state, picks its loads by a limit of 192 MiB) and, for the sum of squares, against the
     oracle's compensated sum of the same elements."""
     lib = _lib()
     above, below = (256 << 20) // 4 + 1, (256 << 20) // 4 - 131072 - 7
