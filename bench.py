@@ -356,7 +356,7 @@ def main() -> int:
                     help="the workload's parameters in this dtype instead of its own (gradients keep theirs); "
                          "bf16/fp16 parameters get fp32 masters")
     ap.add_argument("--chunk-elems", type=int, default=None, metavar="N",
-                    help="AdamW(chunk_elems=N): elements per pass-2 work-group (a multiple of 512; default 1,024)")
+                    help="AdamW(chunk_elems=N): elements per entry of pass 2's chunk table (a multiple of 512; default 1,024)")
     ap.add_argument("--alloc-rounds", type=int, default=0, metavar="R",
                     help="after the benchmark line's measurement, release the workload and build it again from "
                          "fresh allocations R times in this process, timing both passes in each round (the spread "

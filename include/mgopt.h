@@ -109,9 +109,9 @@ typedef struct mgopt_plan mgopt_plan;
  * dispatch torch builds per call in torch/optim/adam.py:139-212 _init_group
  * and in _foreach_norm's tensor lists, clip_grad.py:85-96): pass 2 (the AdamW
  * update) works in chunks of chunk_elems elements, which must be a positive
- * multiple of 512, each split over one or more work-groups; pass 1 (the norm) in chunks of its own.  steps_dev is a
- * caller-owned float[n_tensors] holding each tensor's AdamW step count
- * (torch/optim/adam.py:168-176 state["step"]). */
+ * multiple of 512, each split over one or more work-groups; pass 1 (the norm)
+ * in chunks of its own.  steps_dev is a caller-owned float[n_tensors] holding
+ * each tensor's AdamW step count (torch/optim/adam.py:168-176 state["step"]). */
 MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensors, int32_t n_groups,
                                 float* steps_dev, int64_t chunk_elems, mgopt_plan** out);
 
@@ -122,9 +122,9 @@ MGOPT_API int64_t mgopt_plan_num_chunks(const mgopt_plan* plan);
 
 /* 1 when the plan runs a step as three kernels (a plan of at most 2,097,152
  * elements, no empty tensor, with optimizer state no tensor of more than 256
- * pass-2 chunks, MGOPT_FOLD not "0" in the environment at creation; MGOPT_FOLD=1 lifts the
- * two size limits for plans of up to 67,108,864 elements): pass 1 finalizes
- * in its last work-group and pass 2 forms the step counts and constants
+ * pass-2 chunks, MGOPT_FOLD not "0" in the environment at creation;
+ * MGOPT_FOLD=1 lifts the two size limits for plans of up to 67,108,864
+ * elements): pass 1 finalizes in its last work-group and pass 2 forms the step counts and constants
  * itself; 0 for the five-kernel form (pass 1, finalize, prologue, pass 2,
  * scaler); -1 for NULL.  Both forms give the same results.  No reference
  * counterpart. */
@@ -219,16 +219,14 @@ MGOPT_API int mgopt_plan_flags(mgopt_plan* plan, int* out);
 /* The gradient L2 norm of one contiguous gradient buffer of n elements (a
  * flat gradient arena), with the outputs, scaling and arithmetic of
  * mgopt_grad_norm.  It sums the same chunks (of at most 131,072 elements,
- * fewer on small buffers) in the same order as mgopt_grad_norm on a plan holding that buffer as its one tensor in the
- * five-kernel form (a plan of more than 2,097,152 elements, or any plan made
- * with MGOPT_FOLD=0 in the environment), and is bit-identical to it there; a
- * plan of at most 2,097,152 elements runs the three-kernel form, whose
- * 16,384-element chunks group the fp64 partial sums differently, so the two
- * can differ in the last bits of the fp64 total.  Allocates nothing: its
- * partial sums live in a static 1 MiB device array that each GPU holds until
+ * down to 16,384 on smaller buffers) in the same order as mgopt_grad_norm on a
+ * plan holding that buffer as its one tensor, and is bit-identical to it; only
+ * a plan of more than 67,076,096 elements that MGOPT_FOLD=1 keeps in the
+ * three-kernel form, whose chunks are always 16,384 long, can differ in the
+ * last bits of the fp64 total.  Allocates nothing: its partial sums live in a static 1 MiB device array that each GPU holds until
  * the process ends, so n is at most 8,589,934,592 (65,536 chunks of 131,072
- * elements; larger n returns MGOPT_E_LIMIT).  Runs on the current device.  Calls that overlap on
- * one GPU share that array and race.  No counterpart in the reference: it is
+ * elements; larger n returns MGOPT_E_LIMIT).  Runs on the current device.
+ * Calls that overlap on one GPU share that array and race.  No counterpart in the reference: it is
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc). */
 MGOPT_API int mgopt_grad_norm_noalloc(const void* grads_dev, int32_t grad_dtype, int64_t n, const float* scale_dev,

@@ -220,9 +220,10 @@ class AdamW(torch.optim.Optimizer):
         .grad during the step (the reference leaves them in .grad;
         train.py never reads them after the step, so this is off by default).
     chunk_elems: elements per entry of pass 2's chunk table (a multiple of
-        512), split over work-groups of 256 elements; by default 2,048 for a set small enough for the three-kernel step at that
-        chunk (at most 2,097,152 elements, no tensor of more than 256 chunks),
-        1,024 otherwise.
+        512), split over work-groups of 256 elements (one work-group each in
+        the three-kernel step); by default 2,048 for a set small enough for
+        the three-kernel step at that chunk (at most 2,097,152 elements, no
+        tensor of more than 256 chunks), 1,024 otherwise.
     state_layout: "rows" (default) keeps each parameter's fp32 master,
         exp_avg and exp_avg_sq rows side by side in memory when its row
         length (the smallest product of trailing dimensions that is a
@@ -309,8 +310,8 @@ class AdamW(torch.optim.Optimizer):
     def _get_engine(self) -> _Engine:
         if self._engine is None:
             if torch.cuda.is_current_stream_capturing():
-                # creating the engine allocates device and pinned host memory
-                # and uploads its tables, none of which a graph can record
+                # creating the engine allocates device memory and uploads its
+                # tables, neither of which a graph can record
                 raise RuntimeError("this optimizer has not stepped yet: run one step outside graph capture "
                                    "before capturing")
             capturable = bool(self.defaults.get("capturable")) or any(g.get("capturable") for g in self.param_groups)

@@ -43,7 +43,8 @@ class _GradPlan:
             d.group = 0
             d.grad_dtype = code
             d.lowp_dtype = N.NONE
-        # elements per work-group of the in-place scaling: 4 KB of gradients (mgopt.hip, scale_grads_kernel)
+        # a chunk-table entry per 4 KB of gradients, four work-groups of the in-place scaling (mgopt.hip,
+        # scale_grads_kernel)
         chunk = 1024 if any(code == N.F32 for _, code in sets) else 2048
         plan = ctypes.c_void_p()
         with torch.cuda.device(index):

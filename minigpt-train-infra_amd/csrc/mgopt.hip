@@ -45,8 +45,8 @@ constexpr int kBlock = 512;          // work-group size of pass 1, finalize and 
 // order: work-group b takes the elements from 256 b on, so the eight XCDs walk
 // one window together, a KB of each stream each in turn.  Of a work-group's three
 // waves the first gives each lane one 4-element group and the others retire
-// at once: 32 wave slots a CU let ten work-groups in, and ten to sixteen waves
-// of memory traffic per CU are what HBM takes best.  Whole steps, one process, same
+// at once.  Why those help was not taken apart; the form was chosen because it
+// measures best.  Whole steps, one process, same
 // buffers, in us (ms from GPT-1.3B on):
 //                                    GPT 4x512  GPT-2-small  fp32, grads  GPT-1.3B  2.5e9 in 20k  2.8e9 Qwen3-
 //   threads, elements, order         bf16       fp16 grads   written back bf16      ragged        8B shapes
@@ -61,9 +61,7 @@ constexpr int kBlock = 512;          // work-group size of pass 1, finalize and 
 //   320, 512, dispatch order         183        548          709          6.16      11.87         13.34
 //   512, 1,024, dispatch order       195        562          751          6.03      11.16         12.90
 // (the first row from another process).  128 elements per work-group ran 3-30 %
-// slower.  64-thread work-groups held at 14 a CU by reserved LDS measured as
-// 192 over 256 do; held at 8, 14 % slower, at 10 9 %, at 26 2 %.  XCDs taking
-// turns by 4 KB up to 4 MB instead of 1 KB: 0-8 % slower.
+// slower.  XCDs taking turns by 4 KB up to 4 MB instead of 1 KB: 0-8 % slower.
 constexpr int kAdamBlock = 192;      // work-group size of pass 2
 constexpr int64_t kSubElems = 256;   // elements per work-group of pass 2
 constexpr uint32_t kMaxSubShift = 8; // at most 256 work-groups per entry of the chunk table (a user's longer chunks)
@@ -1487,8 +1485,8 @@ int dtype_size(int32_t dt) {
 // ---------------------------------------------------------------------------
 
 // Partials of mgopt_grad_norm_noalloc, one per chunk of at most 131,072
-// elements: 1 MiB, so one call covers at most 65,536 x 131,072 = 8,589,934,592 elements.  Each
-// GPU the library runs on holds its own copy until the process ends, and every
+// elements: 1 MiB, so one call covers at most 65,536 x 131,072 = 8,589,934,592
+// elements.  Each GPU the library runs on holds its own copy until the process ends, and every
 // call on that GPU shares it (calls that overlap on one GPU race).  Every slot
 // a call reads is written by the same call, so nothing needs clearing.
 constexpr int64_t kScratchPartials = 65536;
@@ -1639,7 +1637,12 @@ MGOPT_API int mgopt_plan_create(const mgopt_tensor_desc* descs, int32_t n_tensor
     for (auto& c : P->classes) {
         c.cached_from = c.norm_count;
         c.first = 0;
-        // a larger set: its last gradients
+        // a larger set: its last gradients.  Without a pass 2 they would not
+        // be read from the cache (kClipCachedBytes).  With several classes,
+        // whose launches follow each other in both passes, nothing is cached,
+        // as before the rule: the gradients of the class that pass 1 reads
+        // last would serve if pass 2 began with that class, which has not been
+        // measured.
         if (P->grad_bytes > cache_limit && (!with_state || P->classes.size() > 1)) continue;
         const int64_t size = dtype_size(c.grad_dtype);
         auto span = std::upper_bound(norm_spans.begin(), norm_spans.end(), c.norm_begin + c.norm_count - 1,

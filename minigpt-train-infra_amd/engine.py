@@ -232,8 +232,8 @@ class _Engine:
         self.hp_key: list[tuple] | None = None
         self.hp_raw: list[tuple] | None = None
         # capturable: the kernels read the group records from a fixed device
-        # buffer (refreshed from param_groups by asynchronous copies outside
-        # any capture), the bias-correction table has a fixed size, and once a
+        # buffer (refreshed from param_groups by a small kernel outside any
+        # capture), the bias-correction table has a fixed size, and once a
         # step was captured the plan's device tables may not be replaced
         self.capturable = capturable
         self.captured = False

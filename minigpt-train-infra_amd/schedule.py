@@ -47,7 +47,7 @@ def build_adamw_param_groups(model: torch.nn.Module, weight_decay: float) -> lis
 def set_optimizer_lr(optimizer: torch.optim.Optimizer, lr: float) -> None:
     """Writes one learning rate into every group (src/minigpt/optim.py:67-71).
     A capturable AdamW of this package also gets the value into the device
-    records a captured step reads (an asynchronous copy)."""
+    records a captured step reads (written by a kernel, in stream order)."""
     for group in optimizer.param_groups:
         group["lr"] = lr
     refresh = getattr(optimizer, "refresh_hparams", None)

@@ -26,6 +26,7 @@ GROUPS, SHORTEST = 2048, 16384      # chunks a set is split into, shortest chunk
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("sizes", [
+    (2_097_152,),                                       # the largest whose pass 1 finalizes
     (2_097_153,),                                       # the smallest set with a finalize of its own
     (SHORTEST * (GROUPS - 1),),                         # the last with the shortest chunks, all whole
     (SHORTEST * GROUPS * 2 - SHORTEST * 2,),            # one chunk short of the next length
